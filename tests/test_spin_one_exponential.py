@@ -1,0 +1,57 @@
+"""The spin-one step exponential at the edges of its series (largest
+eigenvalue 0.015 and 1/4) and of its squarings, and where squaring is kept
+unitary, against the eigendecomposition of the generator."""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+
+import spinsim_amd as ss
+
+EPS = 2.0 ** -52
+DEVICES = [ss.Device.CPU_SINGLE, pytest.param(ss.Device.ROCM, marks=pytest.mark.gpu)]
+METHODS = [ss.ExponentiationMethod.LIE_TROTTER, ss.ExponentiationMethod.LIE_TROTTER_8]
+
+
+def generator(g):
+    x, y, z, q, u1, u2, v1, v2 = list(g) + [0.0] * (8 - len(g))
+    a, b = x - 1j * y + v1 - 1j * v2, x - 1j * y - v1 + 1j * v2
+    m = np.diag([z + q / 3, -2 * q / 3, q / 3 - z]).astype(complex)
+    m[0, 1], m[1, 2], m[0, 2] = a / math.sqrt(2), b / math.sqrt(2), u1 - 1j * u2
+    return np.tril(m.conj().T, -1) + m
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("method", METHODS)
+def test_step_exponential(device, method):
+    n = 8 if method is METHODS[1] else 4
+    src = ("__device__ void get_field(double t, const double* s, double* f)\n"
+           "{ for (int k = 0; k < %d; ++k) f[k] = s[k]; }" % n)
+    sim = ss.Simulator(src, ss.SpinQuantumNumber.ONE, device=device, exponentiation_method=method,
+                       use_rotating_frame=False, integration_method=ss.IntegrationMethod.EULER)
+    rng = np.random.default_rng(5)
+    radii = [0.0, 1e-12, 1e-3, 0.0149, 0.0151, 0.1, 0.249, 0.251, 0.49, 0.51, 3.0, 40.0, 1e6, 1e9]
+    for rho in radii:
+        for _ in range(4):
+            g = rng.normal(size=n)
+            g *= rho / np.abs(np.linalg.eigvalsh(generator(g))).max()
+            u = sim.evaluate(0.0, 1.5, 1.0, 1.0, [1, 0, 0], list(g)).time_evolution[0]
+            # rounding of p, q, the entries and each of the squares, which all
+            # scale with the angle (at most; beyond 8 squares the result is
+            # made unitary again after each)
+            bound = 32 * EPS * (1 + min(rho, 2.0 ** 22))
+            assert np.abs(u.conj().T @ u - np.eye(3)).max() <= bound, rho
+            if rho <= 40:
+                w, v = np.linalg.eigh(generator(g))
+                assert np.abs(u - (v * np.exp(-1j * w)) @ v.conj().T).max() <= bound, rho
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("value", [math.inf, math.nan])
+def test_non_finite_field(device, value):
+    src = "__device__ void get_field(double t, const double* s, double* f) { f[0] = s[0]; f[3] = 1; }"
+    sim = ss.Simulator(src, ss.SpinQuantumNumber.ONE, device=device)
+    u = sim.evaluate(0.0, 1.5, 1.0, 1.0, [1, 0, 0], [value]).time_evolution
+    assert not np.isfinite(u).any()
