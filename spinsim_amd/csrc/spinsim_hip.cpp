@@ -1207,19 +1207,23 @@ int ss_time_evolution_events(void* start_event, void* stop_event)
 
 uint64_t ss_source_hash(void)
 {
-    uint64_t h = 1469598103934665603ull;
-    h = fnv1a(ss_src_args, h);
-    h = fnv1a(ss_src_complex, h);
-    h = fnv1a(ss_src_prelude, h);
-    h = fnv1a(ss_src_integrator, h);
-    // the compiler options and the hipRTC version make a different code
-    // object from the same text
-    for (const char* o : kRtcOptions) h = fnv1a(o, fnv1a("\x1f", h));
-    int major = 0, minor = 0;
-    hiprtcVersion(&major, &minor);
-    char ver[32];
-    snprintf(ver, sizeof(ver), "hiprtc %d.%d", major, minor);
-    return fnv1a(ver, h);
+    // (the text and the compiler do not change within a process)
+    static const uint64_t hash = [] {
+        uint64_t h = 1469598103934665603ull;
+        h = fnv1a(ss_src_args, h);
+        h = fnv1a(ss_src_complex, h);
+        h = fnv1a(ss_src_prelude, h);
+        h = fnv1a(ss_src_integrator, h);
+        // the compiler options and the hipRTC version make a different code
+        // object from the same text
+        for (const char* o : kRtcOptions) h = fnv1a(o, fnv1a("\x1f", h));
+        int major = 0, minor = 0;
+        hiprtcVersion(&major, &minor);
+        char ver[32];
+        snprintf(ver, sizeof(ver), "hiprtc %d.%d", major, minor);
+        return fnv1a(ver, h);
+    }();
+    return hash;
 }
 
 void ss_free(void* p) { std::free(p); }
