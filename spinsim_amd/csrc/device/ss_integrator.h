@@ -179,16 +179,15 @@ static __device__ __forceinline__ void ss_square_hypercubes(ss_cd a[SS_D][SS_D])
 // ---- matrix exponentials of -i g.J ----------------------------------------
 #if SS_DIM == 2 && SS_DIRECT_EXPO
 // matrix_exponential_analytic, spinsim/__init__.py:1617-1641:
-// exp(-i g.sigma/2) = cos(r/2) I - i (sin(r/2)/r) g.sigma, r = |g|, as the
-// first column (b0, b1) of its residual, exp - I.
+// exp(-i g.sigma/2) = cos(r/2) I - i (sin(r/2)/r) g.sigma, r2 = r^2 = |g|^2, as
+// the first column (b0, b1) of its residual, exp - I.
 // Both scalars are even in r, so for r < 1/4 they come from their Taylor
 // series in u = r^2/4 (to u^5: truncation below 3e-20 relative) -- no square
 // root, division or normalised axis; beyond, cos_exp_m1(r/2, 0) =
 // -2 sin^2(r/4) and sin(r/2) from one sincos of r/4.
-static __device__ __forceinline__ void ss_expo_su2_m1(const double g[SS_FIELD_LEN], ss_cd& b0, ss_cd& b1)
+static __device__ __forceinline__ void ss_expo_su2_m1(const double g[SS_FIELD_LEN], double r2, ss_cd& b0, ss_cd& b1)
 {
     const double x = g[0], y = g[1], z = g[2];
-    const double r2 = x * x + y * y + z * z;
     double c, sr;  // cos(r/2) - 1 and sin(r/2)/r
     if (r2 < 0.0625) {
         const double u = 0.25 * r2;
@@ -616,12 +615,12 @@ static __device__ __forceinline__ void ss_call_field(double t, const double* swe
 static __device__ __forceinline__ void ss_frame(double f[SS_FIELD_LEN], double rot, ss_cd w)
 {
 #if SS_ROT
-#if SS_DIM == 2
-    const ss_cd x = ss_mul(ss_c(f[0], f[1]), ss_conj(w));
-    f[2] = f[2] - 2.0 * rot;
-#else
-    const ss_cd x = ss_mul(ss_c(f[0], f[1]), ss_conj(w));
-    f[2] = f[2] - rot;
+    // (a callback that leaves the y field alone is common, and its zero is a
+    // constant here)
+    const ss_cd x = __builtin_constant_p(f[1]) && f[1] == 0.0 ? ss_c(f[0] * w.x, -f[0] * w.y)
+                                                              : ss_mul(ss_c(f[0], f[1]), ss_conj(w));
+    f[2] = f[2] - (SS_DIM == 2 ? 2.0 : 1.0) * rot;
+#if SS_DIM == 3
 #if SS_LIE == 8
     // transform_frame_spin_one_rotating_8, :586-596: U1/U2 turn at twice the
     // frame rate, V1/V2 at the frame rate
@@ -712,16 +711,70 @@ static __device__ __forceinline__ void ss_append(const double g[SS_FIELD_LEN], s
 // column: with U = I + a, a's column (p, q) and the step's residual B = E - I,
 // a <- a + B (I + a) takes four complex products where the full 2x2 product
 // takes eight, and rounds at the size of a, not of 1.
-static __device__ __forceinline__ void ss_append_su2(const double g[SS_FIELD_LEN], ss_cd& p, ss_cd& q)
+static __device__ __forceinline__ void ss_append_column(ss_cd b0, ss_cd b1, ss_cd& p, ss_cd& q)
 {
-    ss_cd b0, b1;
-    ss_expo_su2_m1(g, b0, b1);
     const ss_cd u = ss_c(1.0 + p.x, p.y);
     const ss_cd np = ss_mac(ss_mac(p, b0, u), ss_c(-b1.x, b1.y), q);
     const ss_cd nq = ss_mac(ss_mac(q, b1, u), ss_conj(b0), q);
     p = np;
     q = nq;
 }
+
+#if SS_DIRECT_EXPO
+// exp(-i g.sigma/2) = cos(r/2) (I - i tau g.sigma), tau = tan(r/2)/r.  Steps of
+// r <= 0.018 are applied without the factor cos(r/2): V = -i tau g.sigma needs
+// one series (to r^6; the first term left out is below 1e-20 of the operator)
+// and, its diagonal being imaginary, 12 multiply-adds where the two series and
+// the general product take 11 more instructions.  The chunk's product comes
+// out a positive multiple of a special unitary matrix, and ss_su2_normalise
+// divides by its norm once per chunk.  Larger steps take the exponential.
+#define SS_SU2_R2_SMALL 3.24e-4
+// Steps after which the product is normalised in any case, so that the residual
+// stays of the operator's size: a small step grows the product by at most
+// 1 / cos(0.009) per exponential, 1,024 steps of two by 9%.
+#define SS_SU2_BLOCK 1024
+
+static __device__ __forceinline__ void ss_append_su2(const double g[SS_FIELD_LEN], ss_cd& p, ss_cd& q)
+{
+    const double r2 = g[0] * g[0] + g[1] * g[1] + g[2] * g[2];
+    if (r2 <= SS_SU2_R2_SMALL) {
+        const double tau = fma(r2, fma(r2, fma(r2, 17.0 / 40320, 1.0 / 240), 1.0 / 24), 0.5);
+        const double x = tau * g[0], y = tau * g[1], z = tau * g[2];
+        // a += V (I + a), V's first column (-i z, y - i x)
+        const double ux = 1.0 + p.x;
+        const double px = fma(z, p.y, fma(-y, q.x, fma(x, q.y, p.x)));
+        const double py = fma(-z, ux, fma(-y, q.y, fma(-x, q.x, p.y)));
+        const double qx = fma(y, ux, fma(x, p.y, fma(-z, q.y, q.x)));
+        const double qy = fma(y, p.y, fma(-x, ux, fma(z, q.x, q.y)));
+        p = ss_c(px, py);
+        q = ss_c(qx, qy);
+    } else {
+        ss_cd b0, b1;
+        ss_expo_su2_m1(g, r2, b0, b1);
+        ss_append_column(b0, b1, p, q);
+    }
+}
+
+// The column (1 + p, q) over its norm: 1/sqrt(1 + d) - 1 = -d / (s (1 + s)),
+// s = sqrt(1 + d), d = |1 + p|^2 + |q|^2 - 1.
+static __device__ __forceinline__ void ss_su2_normalise(ss_cd& p, ss_cd& q)
+{
+    const double d = fma(p.x, p.x + 2.0, p.y * p.y) + fma(q.x, q.x, q.y * q.y);
+    const double s = sqrt(1.0 + d);
+    const double f = -d / (s * (1.0 + s));
+    p.x = fma(f, 1.0 + p.x, p.x);
+    p.y = fma(f, p.y, p.y);
+    q.x = fma(f, q.x, q.x);
+    q.y = fma(f, q.y, q.y);
+}
+#else
+static __device__ __forceinline__ void ss_append_su2(const double g[SS_FIELD_LEN], ss_cd& p, ss_cd& q)
+{
+    ss_cd b0, b1;
+    ss_expo_su2_m1(g, b0, b1);
+    ss_append_column(b0, b1, p, q);
+}
+#endif
 
 static __device__ __forceinline__ void ss_su2_expand(ss_cd p, ss_cd q, ss_cd u[2][2])
 {
@@ -1052,23 +1105,37 @@ static __device__ __forceinline__ void ss_mixed_to_u(const double gsum[SS_LIE], 
 // t' - t is the exact difference of the rounded sample offsets the reference
 // forms, so w follows exp(i r t_rel) of those offsets to ~1e-15 over a
 // chunk; it is re-anchored with sincos at the start of every lane's chunk.
+// t is the sample's time, t_rel its offset from the coarse step's start.
 struct ss_wind {
     ss_cd w;
-    double t_rel;
+    double t, t_rel;
 };
-static __device__ __forceinline__ void ss_wind_advance(ss_wind& s, double t_rel_next, ss_cd step, double r,
+static __device__ __forceinline__ void ss_wind_advance(ss_wind& s, double t_next, double tc, ss_cd step, double r,
                                                        double dt)
 {
+    const double t_rel = t_next - tc;
 #if SS_ROT
-    const double eps = r * ((t_rel_next - s.t_rel) - dt);
+    const double eps = r * ((t_rel - s.t_rel) - dt);
     s.w = ss_mul(ss_mul(s.w, step), ss_c(1.0, eps));
 #else
     (void)step;
     (void)r;
     (void)dt;
 #endif
-    s.t_rel = t_rel_next;
+    s.t = t_next;
+    s.t_rel = t_rel;
 }
+static __device__ __forceinline__ ss_wind ss_wind_start(double t, double tc, double r)
+{
+    ss_wind s;
+    s.t = t;
+    s.t_rel = t - tc;
+    s.w = ss_winding(r, s.t_rel);
+    return s;
+}
+
+// Spin-half products that are normalised after every SS_SU2_BLOCK steps.
+#define SS_NORMALISED_BLOCKS (SS_DIM == 2 && SS_PREC == 0 && SS_DIRECT_EXPO)
 
 // `count` fine steps starting at fine index j0 of the coarse step starting at
 // tc; u (initially identity) accumulates them.  The fine time is advanced by
@@ -1103,58 +1170,68 @@ static __device__ __forceinline__ void ss_integrate(ss_cd u[SS_D][SS_D], int j0,
 #define SS_APPEND(g) ss_append(g, u)
 #endif
     if (count <= 0) return;
-    ss_wind wa, wb;
-    wa.t_rel = (tf + off_a) - tc;
     const double frot = SS_FRAME_M * rot;
-    wa.w = ss_winding(frot, wa.t_rel);
-    wb.t_rel = (tf + off_b) - tc;
+    ss_wind wa = ss_wind_start(tf + off_a, tc, frot);
 #if SS_METHOD != 1
-    wb.w = ss_winding(frot, wb.t_rel);
+    ss_wind wb = ss_wind_start(tf + off_b, tc, frot);
 #endif
     const ss_cd step = ss_winding(frot, dt);
-#pragma unroll 1
-    for (int j = 0; j < count; ++j) {
-        double fa[SS_FIELD_LEN], g[SS_FIELD_LEN];
-#if SS_METHOD == 1
-        // euler (midpoint sample), :758-791
-        ss_call_field(wa.t_rel + tc, sweep, fa, ctx);
-        ss_frame(fa, rot, wa.w);
-#pragma unroll
-        for (int k = 0; k < SS_FIELD_LEN; ++k) g[k] = dt * fa[k];
-        SS_APPEND(g);
-#else
-        double fb[SS_FIELD_LEN];
-        ss_call_field(wa.t_rel + tc, sweep, fa, ctx);
-        ss_call_field(wb.t_rel + tc, sweep, fb, ctx);
-        ss_frame(fa, rot, wa.w);
-        ss_frame(fb, rot, wb.w);
-        // both exponents first, so the samples are dead before the exponentials
-        double g2[SS_FIELD_LEN];
 #if SS_METHOD == 0
-        // magnus_cf4, :655-686
-#pragma unroll
-        for (int k = 0; k < SS_FIELD_LEN; ++k) {
-            g[k] = dt * (SS_W0 * fa[k] + SS_W1 * fb[k]);
-            g2[k] = dt * (SS_W1 * fa[k] + SS_W0 * fb[k]);
-        }
+    const double k0 = dt * SS_W0, k1 = dt * SS_W1;
+#endif
+#if SS_NORMALISED_BLOCKS
+#pragma unroll 1
+    for (int left = count; left > 0; left -= SS_SU2_BLOCK) {
+        const int block = left < SS_SU2_BLOCK ? left : SS_SU2_BLOCK;
 #else
-        // heun (half step), :724-752
+    {
+        const int block = count;
+#endif
+#pragma unroll 1
+        for (int j = 0; j < block; ++j) {
+            double fa[SS_FIELD_LEN], g[SS_FIELD_LEN];
+#if SS_METHOD == 1
+            // euler (midpoint sample), :758-791
+            ss_call_field(wa.t, sweep, fa, ctx);
+            ss_frame(fa, rot, wa.w);
 #pragma unroll
-        for (int k = 0; k < SS_FIELD_LEN; ++k) {
-            g[k] = dt * fa[k] / 2;
-            g2[k] = dt * fb[k] / 2;
-        }
+            for (int k = 0; k < SS_FIELD_LEN; ++k) g[k] = dt * fa[k];
+            SS_APPEND(g);
+#else
+            double fb[SS_FIELD_LEN];
+            ss_call_field(wa.t, sweep, fa, ctx);
+            ss_call_field(wb.t, sweep, fb, ctx);
+            ss_frame(fa, rot, wa.w);
+            ss_frame(fb, rot, wb.w);
+            // both exponents first, so the samples are dead before the exponentials
+            double g2[SS_FIELD_LEN];
+#if SS_METHOD == 0
+            // magnus_cf4, :655-686
+#pragma unroll
+            for (int k = 0; k < SS_FIELD_LEN; ++k) {
+                g[k] = fma(k0, fa[k], k1 * fb[k]);
+                g2[k] = fma(k0, fb[k], k1 * fa[k]);
+            }
+#else
+            // heun (half step), :724-752
+#pragma unroll
+            for (int k = 0; k < SS_FIELD_LEN; ++k) {
+                g[k] = dt * fa[k] / 2;
+                g2[k] = dt * fb[k] / 2;
+            }
 #endif
-        SS_APPEND(g);
-        SS_APPEND(g2);
+            SS_APPEND(g);
+            SS_APPEND(g2);
 #endif
-        tf += dt;
-        if (j + 1 < count) {
-            ss_wind_advance(wa, (tf + off_a) - tc, step, frot, dt);
+            tf += dt;
+            ss_wind_advance(wa, tf + off_a, tc, step, frot, dt);
 #if SS_METHOD != 1
-            ss_wind_advance(wb, (tf + off_b) - tc, step, frot, dt);
+            ss_wind_advance(wb, tf + off_b, tc, step, frot, dt);
 #endif
         }
+#if SS_NORMALISED_BLOCKS
+        ss_su2_normalise(su_p, su_q);
+#endif
     }
 #if SS_PREC != 0
     ss_mixed_to_u(gsum, bres, u);
@@ -2012,26 +2089,23 @@ ss_batch_adjoint_kernel(ss_adjoint_args a)
     for (int k = 0; k + 1 < n_fine; ++k) tf += dt;
     const double frot = SS_FRAME_M * rot;
     const ss_cd back = ss_conj(ss_winding(frot, dt));
-    ss_wind wa, wb;
-    wa.t_rel = (tf + off_a) - tc;
-    wa.w = ss_winding(frot, wa.t_rel);
-    wb.t_rel = (tf + off_b) - tc;
+    ss_wind wa = ss_wind_start(tf + off_a, tc, frot);
 #if SS_METHOD != 1
-    wb.w = ss_winding(frot, wb.t_rel);
+    ss_wind wb = ss_wind_start(tf + off_b, tc, frot);
 #endif
 #pragma unroll 1
     for (int j = n_fine - 1; j >= 0; --j) {
         if (j < n_fine - 1) {
             tf -= dt;
-            ss_wind_advance(wa, (tf + off_a) - tc, back, frot, -dt);
+            ss_wind_advance(wa, tf + off_a, tc, back, frot, -dt);
 #if SS_METHOD != 1
-            ss_wind_advance(wb, (tf + off_b) - tc, back, frot, -dt);
+            ss_wind_advance(wb, tf + off_b, tc, back, frot, -dt);
 #endif
         }
         double fa[SS_FIELD_LEN], g1[SS_FIELD_LEN], d1[SS_LIE], dfa[SS_LIE], lab[4];
         const double tra = wa.t_rel;
         const ss_cd wa_w = wa.w;
-        ss_call_field(tra + tc, sweep, fa, &ctx);
+        ss_call_field(wa.t, sweep, fa, &ctx);
         ss_frame(fa, rot, wa_w);
 #pragma unroll
         for (int k = 0; k < SS_LIE; ++k) d1[k] = 0.0;
@@ -2045,12 +2119,12 @@ ss_batch_adjoint_kernel(ss_adjoint_args a)
         if (z_control) dz_mid += tra * (dfa[0] * fa[1] - dfa[1] * fa[0]) - dfa[2];
 #endif
         ss_unframe(dfa, wa_w, lab);
-        ss_scatter_sample(a, &ctx, tra + tc, lab, win, base, grad_row, mo);
+        ss_scatter_sample(a, &ctx, wa.t, lab, win, base, grad_row, mo);
 #else
         double fb[SS_FIELD_LEN], g2[SS_FIELD_LEN], d2[SS_LIE], dfb[SS_LIE];
         const double trb = wb.t_rel;
         const ss_cd wb_w = wb.w;
-        ss_call_field(trb + tc, sweep, fb, &ctx);
+        ss_call_field(wb.t, sweep, fb, &ctx);
         ss_frame(fb, rot, wb_w);
 #pragma unroll
         for (int k = 0; k < SS_LIE; ++k) d2[k] = 0.0;
@@ -2087,9 +2161,9 @@ ss_batch_adjoint_kernel(ss_adjoint_args a)
                       trb * (dfb[0] * fb[1] - dfb[1] * fb[0]) - dfb[2];
 #endif
         ss_unframe(dfa, wa_w, lab);
-        ss_scatter_sample(a, &ctx, tra + tc, lab, win, base, grad_row, mo);
+        ss_scatter_sample(a, &ctx, wa.t, lab, win, base, grad_row, mo);
         ss_unframe(dfb, wb_w, lab);
-        ss_scatter_sample(a, &ctx, trb + tc, lab, win, base, grad_row, mo);
+        ss_scatter_sample(a, &ctx, wb.t, lab, win, base, grad_row, mo);
 #endif
     }
 #if SS_ROT
