@@ -1415,6 +1415,7 @@ static __device__ __forceinline__ void ss_te_item(const ss_te_args& a, long long
 // coarse step for every row).
 extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_kernel(ss_te_args a)
 {
+    ss_trig_load();
     const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     if (wave >= a.items) return;  // whole waves only
     ss_ctx ctx;
@@ -1429,6 +1430,7 @@ extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_kernel(ss_te_args a)
 // fine step of the others.
 extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_phased_kernel(ss_te_args a)
 {
+    ss_trig_load();
     const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     ss_ctx ctx;
     ctx.tables = reinterpret_cast<const ss_table*>(a.tables);
@@ -1451,6 +1453,7 @@ extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_phased_kernel(ss_te_
 // together; every wave leaves once the counter passes the total.
 extern "C" __global__ void SS_KERNEL_ATTR ss_batch_time_evolution_kernel(ss_batch_args a)
 {
+    ss_trig_load();
     const int lane = threadIdx.x & 63;
     const int lanes = a.lanes_per_step;
     const int groups = 64 / lanes;
@@ -1986,6 +1989,7 @@ ss_batch_adjoint_kernel(ss_adjoint_args a)
     // lane's window is ss_adj_windows[k * SS_ADJ_BLOCK + lane], so a wave's
     // accesses to one slot are consecutive doubles, free of LDS bank conflicts
     extern __shared__ double ss_adj_windows[];
+    ss_trig_load();
     const long long row = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     double* win = ss_adj_windows + threadIdx.x;
 #pragma unroll

@@ -1135,6 +1135,14 @@ std::string build_source(const char* field_src, int dim, int method, int expo, i
     int hyper = (number_of_squares + 1) / 2;  // ceil(squares / 2), :1547
     if (number_of_squares <= 0) hyper = 0;
     std::string s;
+    // The sin/cos table goes to LDS for callbacks that evaluate them (two
+    // gathers a step: 1.1e8 spin-half rows 13.51 -> 12.82 ms).  Without, only
+    // the windings of each coarse step read it; and where the adjoint kernel is
+    // specialised for its controls, the 16 KiB would halve its workgroups at
+    // three controls.
+    const bool lds = (std::strstr(field_src, "cos") || std::strstr(field_src, "sin")) &&
+                     !std::strstr(field_src, "SS_ADJ_AXES");
+    if (lds) s += "#define SS_TRIG_LDS 1\n";
     char head[512];
     snprintf(head, sizeof(head),
              "#define SS_DIM %d\n#define SS_LIE %d\n#define SS_METHOD %d\n#define SS_EXPO %d\n"
