@@ -132,14 +132,11 @@ def module_source(field_src, dim, method, expo, rotating, number_of_squares, has
             f"#define SS_EXPO {expo}\n#define SS_ROT {1 if rotating else 0}\n"
             f"#define SS_HYPER {hyper}\n#define SS_CTX {1 if has_context else 0}\n"
             f"#define SS_PREC {precision}\n")
-    # the callback's sin and cos: the table-driven float64 functions, or with
-    # precision fp32 float32 ones with exp as well (ss_prelude.h), as on the GPU
-    if precision == 3:
-        on = "#define sin(x) ss_sin32(x)\n#define cos(x) ss_cos32(x)\n#define exp(x) ss_exp32(x)\n"
-        off = "#undef sin\n#undef cos\n#undef exp\n"
-    else:
-        on = "#define sin(x) ss_sin64(x)\n#define cos(x) ss_cos64(x)\n"
-        off = "#undef sin\n#undef cos\n"
+    # the callback's sin, cos and exp: the table-driven float64 functions, or with
+    # precision fp32 the float32 ones (ss_prelude.h), as on the GPU
+    bits = 32 if precision == 3 else 64
+    on = "".join(f"#define {f}(x) ss_{f}{bits}(x)\n" for f in ("sin", "cos", "exp"))
+    off = "#undef sin\n#undef cos\n#undef exp\n"
     return (head + '#include "host/ss_host_prelude.h"\n#include "device/ss_args.h"\n'
             '#include "device/ss_complex.h"\n#include "device/ss_prelude.h"\n'
             + on + '#line 1 "get_field"\n' + field_src + "\n" + off +
@@ -236,11 +233,11 @@ def f32_eval(fn, x):
 
 
 def f64_eval(fn, x):
-    """The field callbacks' table-driven float64 sin / cos (every precision
-    but "fp32"), host build: fn in ("sin", "cos")."""
+    """The field callbacks' table-driven float64 sin / cos / exp (every precision
+    but "fp32"), host build: fn in ("sin", "cos", "exp")."""
     x = np.ascontiguousarray(np.atleast_1d(np.asarray(x, np.float64)))
     out = np.empty_like(x)
-    _check(host_lib().ss_host_f64_eval(("sin", "cos").index(fn), x.ctypes.data,
+    _check(host_lib().ss_host_f64_eval(("sin", "cos", "exp").index(fn), x.ctypes.data,
                                        out.ctypes.data, x.size), "ss_host_f64_eval")
     return out
 
