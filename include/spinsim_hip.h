@@ -168,13 +168,19 @@ int ss_module_info(const ss_module *m, int *vgprs, int *sgprs, int *scratch_byte
  * dt_out), taken out of the rotating frame.  `dt` is the integration step as
  * evaluate() re-derives it.  sweep: device array read by get_field; tables:
  * device ss_table array or NULL.  lanes_per_step in 1..64: that many lanes
- * share one coarse step; 0 (the default): as many waves as fit on the device
- * at once, with rows dealt in phases of decreasing item length (lanes per
- * step) so all waves finish together; -k (1..64): the same on k waves per
- * SIMD.  u_out: n_coarse*dim*dim complex128. */
+ * share one coarse step; 0 (the default): the lanes ss_default_lanes gives for
+ * the module and the device, or -3 (spin half) or -2 (spin one) in the float32
+ * modes; -k (1..64): k waves per SIMD, with rows dealt in
+ * phases of decreasing item length (lanes per step) so the waves finish
+ * together.  u_out: n_coarse*dim*dim complex128. */
 int ss_time_evolution(const ss_module *m, const double *sweep, double t0, double dt,
                       double dt_out, int64_t n_coarse, double *time_out, double *u_out,
                       const ss_table *tables, int lanes_per_step, ss_stream stream);
+/* Lanes per coarse step of the default launch for n_rows rows of n_fine steps
+ * on `cus` compute units that hold `resident` workgroups each (host only; 1..64,
+ * 1 for invalid arguments).  (No reference counterpart: a launch-planning
+ * query.) */
+int ss_default_lanes(int64_t n_rows, int n_fine, int64_t cus, int64_t resident);
 /* The phase table a phased ss_time_evolution launch on `waves` waves uses
  * (host only): *n_phases phases; phase p starts at coarse row first_row[p]
  * and has items[p] items of 64/lanes[p] rows, each row's fine steps split

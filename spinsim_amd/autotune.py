@@ -1,6 +1,6 @@
 """Launch-shape autotuner for the time-evolution kernels and the batch scans.
 
-Chooses between the phased default launch and a number of lanes sharing one
+Chooses between the default launch, phased launches and a number of lanes sharing one
 coarse step (threads per simulation step), for batches how many rows a wave
 takes per grab of the work counter (the tile of work), and the rows per
 workgroup chunk of the per-simulation state scans, by timing the candidates
@@ -15,8 +15,8 @@ import os
 import statistics
 import threading
 
-# Phased launches timed by tune_lanes: the resident waves, and 1-4 waves per
-# SIMD (fewer, longer items against more waves to hide latency).
+# The default launch and the phased ones on 1-4 waves per SIMD (fewer, longer
+# items against more waves to hide latency), as timed by tune_lanes.
 PHASED_CANDIDATES = [0, -1, -2, -3, -4]
 
 _lock = threading.Lock()
@@ -92,9 +92,9 @@ def time_interleaved(fns: dict, rounds: int = 5, warmup: int = 1):
 
 def tune_lanes(sim, n_coarse: int, n_fine: int, dt: float, dt_out: float, sweep, t0: float = 0.0,
                reps: int = 7, use_cache: bool = True):
-    """Best lanes_per_step for one simulation of this shape (0: phased launch
-    on the resident waves, -k: phased on k waves per SIMD for k = 1..4, else
-    lanes per coarse step); returns (lanes, table)."""
+    """Best lanes_per_step for one simulation of this shape (0: the default
+    launch, -k: phased on k waves per SIMD for k = 1..4, else lanes per coarse
+    step); returns (lanes, table)."""
     import torch
 
     candidates = PHASED_CANDIDATES + lane_candidates(n_fine)

@@ -1369,6 +1369,10 @@ static __device__ __forceinline__ void ss_store(ss_cd u[SS_D][SS_D], double rot,
 
 // ---- GPU kernels (the host build of this text, for the CPU devices, stops here)
 #ifndef SS_HOST
+// What the host reads from a module: its size, 1, or 2 with float32-bulk step
+// operators.
+extern "C" __device__ __attribute__((used)) char ss_module_traits[SS_PREC == 1 || SS_PREC == 3 ? 2 : 1] = {};
+
 // Waves per SIMD the kernels are compiled for at least: the register budget
 // is 512 / waves VGPRs a lane (in 8-register granules).  The time-evolution
 // kernels take what they need (about 230-260 for spin one: their float64
@@ -1424,7 +1428,7 @@ extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_kernel(ss_te_args a)
     ss_te_item(a, wave, 0, 0, &ctx);
 }
 
-// One simulation on the resident waves: wave w takes items w, w + waves,
+// One simulation on a given number of waves: wave w takes items w, w + waves,
 // w + 2 waves, ... of the phase table.  Phases with fewer lanes per row (long
 // items) come first and the finest last, so every wave ends within about one
 // fine step of the others.

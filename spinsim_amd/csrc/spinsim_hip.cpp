@@ -83,8 +83,9 @@ struct ss_module {
     int expo = 0;
     int rotating = 1;
     int device = 0;
-    long long resident_waves = 0;  // phased kernel: waves resident at once
-    long long simds = 0;           // SIMDs of the device (4 per CU)
+    bool float32 = false;          // float32-bulk step operators
+    long long cus = 0;             // compute units of the device
+    long long single_blocks = 0;   // single kernel: workgroups resident per CU
 };
 
 // ---------------------------------------------------------------------------
@@ -1306,16 +1307,24 @@ int ss_module_load(const void* code, size_t code_size, int dim, int method, int 
     if (e == hipSuccess) e = hipModuleGetFunction(&m->phased, m->module, "ss_time_evolution_phased_kernel");
     if (e == hipSuccess) e = hipModuleGetFunction(&m->batch, m->module, "ss_batch_time_evolution_kernel");
     if (e == hipSuccess) e = hipModuleGetFunction(&m->adjoint, m->module, "ss_batch_adjoint_kernel");
+    // (the traits array's size is its content)
+    hipDeviceptr_t traits = nullptr;
+    size_t traits_size = 0;
+    if (e == hipSuccess && hipModuleGetGlobal(&traits, &traits_size, m->module, "ss_module_traits") != hipSuccess) {
+        (void)hipGetLastError();
+        traits_size = 1;
+    }
     int per_cu = 0, cus = 0;
-    if (e == hipSuccess) e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m->phased, 256, 0);
+    if (e == hipSuccess) e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m->single, 256, 0);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->device);
     if (e != hipSuccess) {
         if (m->module) (void)hipModuleUnload(m->module);
         delete m;
         return fail("ss_module_load: %s", hipGetErrorString(e));
     }
-    m->resident_waves = std::max(1LL, (long long)per_cu * cus * 4);
-    m->simds = std::max(1LL, (long long)cus * 4);
+    m->float32 = traits_size == 2;
+    m->cus = std::max(1, cus);
+    m->single_blocks = std::max(1, per_cu);
     *out = m;
     return 0;
 }
@@ -1359,8 +1368,48 @@ int ss_module_info(const ss_module* m, int* vgprs, int* sgprs, int* scratch_byte
     return 0;
 }
 
-// Phase table for a single simulation on `waves` waves.  Candidate lanes per
-// coarse step G are the divisors of n_fine up to 64 (and the powers of two
+// Lanes per coarse step of the default launch (one item per wave, dealt to the
+// device by its own scheduler): the G of the shortest modelled time.  With G
+// lanes a row, W = ceil(N / floor(64 / G)) waves each take
+//     c = 1 + 0.6 ceil(log2 G) + ceil(n_fine / G)
+// fine-step times (set-up of a chunk, its products across lanes, its steps).
+// k workgroups at once on a CU (four waves, one per SIMD) take max(1.6, k) c
+// together: a lone wave waits 1.6 issue times a step.  Full rounds of all
+// resident workgroups come first, then the rest, which overlaps with their end
+// less than fully (1.2).  The four constants were fitted to 126 measured shapes
+// (18 sizes of 40 to 3e5 rows and 1 to 100 steps, seven kernels of 0.1 to 1 us
+// a step): the chosen G is 0.8% slower than the best one on average, 11% at
+// worst, where the launch it replaces (phases over the resident waves) was 28%
+// slower on average and up to 5x.  The float32 modes keep that launch: their
+// chunks round in float32, so their results depend on where rows are cut.
+static int default_lanes(long long n_coarse, int n_fine, long long cus, long long resident)
+{
+    int best = 1;
+    long long last_steps = -1;
+    double best_time = 0;
+    for (int g = 1; g <= std::max(1, std::min(n_fine, 64)); ++g) {
+        const long long steps = ((long long)n_fine + g - 1) / g;
+        if (steps == last_steps) continue;  // the smaller g does as well
+        last_steps = steps;
+        int levels = 0;
+        while ((1 << levels) < g) ++levels;
+        const double c = 1.0 + 0.6 * levels + double(steps);
+        const long long rows = 64 / g;
+        const long long blocks = ((n_coarse + rows - 1) / rows + 3) / 4;
+        const long long full = blocks / (cus * resident), rest = blocks - full * cus * resident;
+        double time = double(full) * c * std::max(1.6, double(resident));
+        if (rest && !full) time += c * std::max(1.6, double((rest + cus - 1) / cus));
+        else if (rest) time += 1.2 * c * std::max(1.6, double(rest) / double(cus));
+        if (g == 1 || time < 0.99 * best_time) {  // (more lanes for a gain of 1%)
+            best = g;
+            best_time = time;
+        }
+    }
+    return best;
+}
+
+// Phase table of the phased launch (lanes_per_step = -k) on `waves` waves.
+// Candidate lanes per coarse step G are the divisors of n_fine up to 64 (and the powers of two
 // when n_fine > 64, where no G gives one step per lane); an
 // item of G covers 64/G rows and costs ceil(n_fine/G) fine steps per lane.
 // Whole rounds (one item per wave) of the coarser G are taken while they fit
@@ -1408,6 +1457,12 @@ static void plan_phases(long long n_coarse, int n_fine, long long waves, ss_te_a
     a->waves = std::max(1LL, std::min(waves, a->items));
 }
 
+int ss_default_lanes(int64_t n_rows, int n_fine, int64_t cus, int64_t resident)
+{
+    if (n_rows < 1 || n_fine < 0 || cus < 1 || resident < 1 || n_rows > (1LL << 40)) return 1;
+    return default_lanes(n_rows, n_fine, cus, resident);
+}
+
 int ss_time_evolution_plan(int64_t n_coarse, int n_fine, int64_t waves, int* n_phases, int* lanes,
                            int64_t* first_row, int64_t* items)
 {
@@ -1453,6 +1508,9 @@ int ss_time_evolution(const ss_module* m, const double* sweep, double t0, double
     a.dt_out = dt_out;
     ss_sample_offsets(m->method, dt, &a.off_a, &a.off_b);
     a.n_fine = n_fine;
+    if (lanes_per_step == 0)
+        lanes_per_step = m->float32 ? (m->dim == 2 ? -3 : -2)
+                                    : default_lanes(n_coarse, n_fine, m->cus, m->single_blocks);
     if (lanes_per_step > 0) {
         const long long groups = 64 / lanes_per_step;
         a.n_phases = 1;
@@ -1461,8 +1519,7 @@ int ss_time_evolution(const ss_module* m, const double* sweep, double t0, double
         a.items = a.phase_items[0];
         a.waves = a.items;
     } else {
-        const long long cap = lanes_per_step < 0 ? (long long)(-lanes_per_step) * m->simds : m->resident_waves;
-        plan_phases(n_coarse, n_fine, cap, &a);
+        plan_phases(n_coarse, n_fine, (long long)(-lanes_per_step) * m->cus * 4, &a);
     }
     const long long blocks = (a.waves + 3) / 4;
     if (blocks > 2147483647LL) return fail("ss_time_evolution: grid too large");

@@ -205,9 +205,9 @@ class Simulator:
 
     Extra keyword arguments: ``samplers`` (for HIP-C field text),
     ``lanes_per_step`` (lanes sharing one coarse step: an int in 1..64;
-    None or 0 for the default launch, which deals the rows to the resident
-    waves in phases of decreasing item length so they finish together; -k
-    for the same on k waves per SIMD; ``"auto"`` to time the candidates on
+    None or 0 for the number a cost model of the launch gives; -k for k
+    waves per SIMD with the rows dealt to them in phases of decreasing item
+    length so they finish together; ``"auto"`` to time the candidates on
     first use of each shape) and
     ``precision``: ``"fp64"`` (default; the reference's arithmetic),
     ``"fp32_bulk"`` -- the higher-order residual exp(A) - I - A of each step
