@@ -192,8 +192,9 @@ int ss_time_evolution_plan(int64_t n_coarse, int n_fine, int64_t waves, int *n_p
 /* Batched time evolution: simulation s owns rows [offsets[s], offsets[s+1])
  * of time_out / u_out and reads sweep row s (sweep + s*sweep_stride).  All
  * arrays are device arrays; offsets has n_sims+1 entries, offsets[n_sims] =
- * total.  counter: one device uint64 the library clears before the launch.
- * grid_blocks = 0 picks a persistent grid for the device.  u_layout: SS_U_FULL
+ * total.  counter: a device uint64, kept for callers; not read or written.
+ * items_per_grab: groups of rows each wave takes (<= 0: 4); grid_blocks > 0
+ * limits the launch to that many workgroups, which then loop over the rows.  u_layout: SS_U_FULL
  * (or SS_U_SU2_FULL, the same store), or SS_U_SU2_COLUMN for a spin-half
  * module (u_out then holds total*2 complex128). */
 int ss_batch_time_evolution(const ss_module *m, const double *sweep, int64_t sweep_stride,

@@ -1,11 +1,11 @@
 """Launch-shape autotuner for the time-evolution kernels and the batch scans.
 
-Chooses between the default launch, phased launches and a number of lanes sharing one
-coarse step (threads per simulation step), for batches how many rows a wave
-takes per grab of the work counter (the tile of work), and the rows per
-workgroup chunk of the per-simulation state scans, by timing the candidates
-on the device with HIP events.  Results are cached per (kernel, shape,
-device) in memory and in a JSON file next to the code-object cache.
+Chooses between the default launch, phased launches and a number of lanes
+sharing one coarse step (threads per simulation step), for batches how many
+groups of rows a wave takes (the tile of work), and the rows per workgroup
+chunk of the per-simulation state scans, by timing the candidates on the
+device with HIP events.  Results are cached per (kernel, shape, device) in
+memory and in a JSON file next to the code-object cache.
 """
 from __future__ import annotations
 

@@ -4,10 +4,9 @@ The reference runs one ``evaluate`` per sweep point (spinsim/__init__.py:993;
 example.py evaluates twice to sweep a bias).  ``BatchPlan`` packs B
 simulations -- each with its own sweep row, start/end time, steps and initial
 state -- into one CSR layout of coarse rows (``offsets[s]`` .. ``offsets[s+1]``
-belong to simulation s), runs them in one persistent time-evolution launch
-that hands out rows from a work counter (uneven durations balance
-themselves), then one state scan per simulation, all stream-ordered and
-capturable in a HIP graph.
+belong to simulation s), runs them in one time-evolution launch over all
+rows (uneven durations balance themselves), then one state scan per
+simulation, all stream-ordered and capturable in a HIP graph.
 """
 from __future__ import annotations
 
@@ -171,8 +170,9 @@ class BatchPlan:
         self.state = torch.empty((total, d), dtype=torch.complex128, device=dev)
         self.lanes = int(lanes_per_step or sim.lanes_per_step or 0)
         if self.lanes <= 0:
-            self.lanes = default_batch_lanes(total, int(nf.max(initial=1)))
-        self.items_per_grab = int(items_per_grab or 4)
+            self.lanes = default_batch_lanes(total, int(nf.max(initial=1)),
+                                             sim.precision in ("fp32", "fp32_bulk"))
+        self.items_per_grab = int(items_per_grab or default_batch_items(total, self.lanes))
         self.grid_blocks = int(grid_blocks)
         self.graph = None
         self.spin_out = (torch.empty((total, 3), dtype=f64, device=dev) if with_spin else None)
@@ -234,7 +234,7 @@ class BatchPlan:
         return self
 
     def capture(self):
-        """Record run() into a HIP graph (the counter is cleared by a kernel)."""
+        """Record run() into a HIP graph."""
         torch = self.sim._torch()
         self.sim._module(self.device)
         self.sim._table_ptr(self.device)
@@ -260,13 +260,28 @@ class BatchPlan:
         return BatchResults(self)
 
 
-def default_batch_lanes(total_rows, max_fine):
-    """Lanes per coarse step for a batch: enough groups to fill the device."""
+def default_batch_lanes(total_rows, max_fine, float32=False):
+    """Lanes per coarse step for a batch: the launch cost model's (256 CUs of
+    three workgroups each).  The float32 modes' results depend on where rows
+    are cut; they keep enough lanes for 32 waves per CU."""
+    if not float32:
+        return int(_native.lib().ss_default_lanes(max(1, int(total_rows)), int(max_fine), 256, 3))
     target = 256 * 4 * 8 * 64
     g = 1
     while g < 64 and 2 * g <= max_fine and total_rows * g < target:
         g *= 2
     return g
+
+
+def default_batch_items(total_rows, lanes):
+    """Groups of rows each wave takes: one until the launch has about two rounds
+    of waves (6,000), then up to four, and up to eight in the longest launches,
+    which spreads a workgroup's set-up over more rows (2e6 rows of 5 steps: 105
+    us at one, 81 at four, 91 at sixteen; 4e5 rows of 10 steps: 36 us at one, 38
+    at four; 1.1e8 rows of 20 steps: 9.05 ms at four, 8.94 at eight, 9.01 at
+    thirty-two)."""
+    waves = -(-int(total_rows) // (64 // lanes))
+    return max(1, min(4, waves // 6000), min(8, waves // 100000))
 
 
 def evaluate_batch(sim, time_start, time_end, time_step_integration, time_step_output, state_init,

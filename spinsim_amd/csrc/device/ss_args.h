@@ -31,9 +31,8 @@ struct ss_te_args {
 };
 
 // Batched launch: simulation s owns coarse rows [offsets[s], offsets[s+1]).
-// Each simulation has its own sweep row, start time and steps.  Work is
-// handed out in units of `items_per_grab` coarse rows from a global counter,
-// so long and short simulations share the machine evenly.
+// Each simulation has its own sweep row, start time and steps.  Each wave takes
+// `items_per_grab` groups of consecutive rows.
 struct ss_batch_args {
     const double* sweep;         // (B, sweep_stride)
     const void* tables;          // ss_table[] or null
@@ -44,7 +43,6 @@ struct ss_batch_args {
     const int* n_fine;           // (B,)
     double* time_out;            // (total,)
     double* u_out;               // (total, d, d) complex128, or (total, 2) with u_layout 1
-    unsigned long long* counter; // work counter, zero before launch
     long long total;             // offsets[B]
     long long n_sims;            // B
     long long sweep_stride;      // doubles per sweep row

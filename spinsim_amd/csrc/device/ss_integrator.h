@@ -1451,44 +1451,42 @@ extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_phased_kernel(ss_te_
     }
 }
 
-// Many simulations in one persistent launch.  Each wave repeatedly takes
-// `items_per_grab` groups' worth of coarse rows from a global counter (one
-// atomic per wave), so simulations with 50x different lengths finish
-// together; every wave leaves once the counter passes the total.
+// Many simulations in one launch.  A workgroup's chunk is 4 * items_per_grab
+// groups of consecutive rows, a quarter for each of its waves; workgroup b takes
+// chunks b, b + grid, ... .  By default there is one workgroup per chunk and
+// the device's own dispatch evens out simulations of different step counts: a
+// shared work counter costs 13 ns a grab (one address for eight XCDs), which
+// bounded launches of short rows (2e6 rows of 5 steps: 154 -> 81 us; 1.5e5 rows
+// of 10 steps, spin one: 59 -> 39 us).
 extern "C" __global__ void SS_KERNEL_ATTR ss_batch_time_evolution_kernel(ss_batch_args a)
 {
     ss_trig_load();
     const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lanes = a.lanes_per_step;
     const int groups = 64 / lanes;
     const int gi = lane / lanes;
     const int rank = lane - gi * lanes;
-    const long long grab = (long long)groups * a.items_per_grab;
+    const long long share = (long long)groups * a.items_per_grab;
 #pragma unroll 1
-    for (;;) {
-        unsigned long long start = 0;
-        if (lane == 0) start = atomicAdd(a.counter, (unsigned long long)grab);
-        start = __shfl(start, 0, 64);
-        if ((long long)start >= a.total) break;
-        // simulation owning the lane's first row of the grab: largest s with
-        // offsets[s] <= row, by bisection; the lane's later rows move it on
-        // by the few starts they pass (a chain of dependent loads per grab
-        // instead of per item)
+    for (long long chunk = blockIdx.x;; chunk += gridDim.x) {
+        const long long start = (chunk * 4 + wave) * share;
+        if (start >= a.total) break;
+        // simulation owning the share's first row: largest s with offsets[s] <=
+        // start, by bisection (the same for the whole wave); each lane's rows
+        // move it on by the starts they pass
         long long lo = 0;
         {
-            const long long row = (long long)start + gi;
             long long hi = a.n_sims;
-            if (gi < groups && row < a.total) {
 #pragma unroll 1
-                while (hi - lo > 1) {
-                    const long long mid = (lo + hi) >> 1;
-                    if (a.offsets[mid] <= row) lo = mid; else hi = mid;
-                }
+            while (hi - lo > 1) {
+                const long long mid = (lo + hi) >> 1;
+                if (a.offsets[mid] <= start) lo = mid; else hi = mid;
             }
         }
 #pragma unroll 1
         for (int it = 0; it < a.items_per_grab; ++it) {
-            const long long row = (long long)start + (long long)it * groups + gi;
+            const long long row = start + (long long)it * groups + gi;
             const bool active = gi < groups && row < a.total;
             if (active) {
 #pragma unroll 1

@@ -1055,11 +1055,6 @@ __global__ void __launch_bounds__(256) interp_kernel(const dev::ss_table* tables
     else dev::ss_interp_sample_axes(&ctx, k, t[i], out + i * axes, axes);
 }
 
-__global__ void zero_counter(unsigned long long* p)
-{
-    if (threadIdx.x == 0) p[0] = 0ull;
-}
-
 // Sustained float64 FMA rate: 8 independent accumulator chains per lane,
 // `iters` rounds of 8 FMAs each; one result per thread keeps the work live.
 __global__ void __launch_bounds__(256) fma_probe_kernel(double* out, long long n, int iters)
@@ -1547,20 +1542,12 @@ int ss_batch_time_evolution(const ss_module* m, const double* sweep, int64_t swe
     if (lanes_per_step > 64) return fail("ss_batch_time_evolution: lanes_per_step must be <= 64");
     if (items_per_grab <= 0) items_per_grab = 4;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (grid_blocks <= 0) {
-        // at least two workgroups (two waves per SIMD) per CU: the occupancy
-        // query reports one for the float64 spin-one kernel (140 VGPRs),
-        // where two run 3% faster on MI355X; extra workgroups of this
-        // persistent kernel only take rows from the same counter
-        int cus = 0, per_cu = 0;
-        SS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->device));
-        SS_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m->batch, 256, 0));
-        grid_blocks = std::max(1, cus * std::max(per_cu, 2));
-    }
     const long long groups = 64 / lanes_per_step;
     const long long per_block = 4LL * groups * items_per_grab;
-    const long long needed = (total + per_block - 1) / per_block;
-    if (grid_blocks > needed) grid_blocks = int(needed);
+    const long long chunks = (total + per_block - 1) / per_block;
+    // one workgroup per chunk, as far as a launch's work-items go (the rest by
+    // the kernel's own loop)
+    const long long grid = std::min(chunks, grid_blocks > 0 ? (long long)grid_blocks : 16777215LL);
     ss_batch_args a;
     a.sweep = sweep;
     a.tables = tables;
@@ -1571,7 +1558,6 @@ int ss_batch_time_evolution(const ss_module* m, const double* sweep, int64_t swe
     a.n_fine = n_fine;
     a.time_out = time_out;
     a.u_out = u_out;
-    a.counter = reinterpret_cast<unsigned long long*>(counter);
     a.total = total;
     a.n_sims = n_sims;
     a.sweep_stride = sweep_stride;
@@ -1583,10 +1569,8 @@ int ss_batch_time_evolution(const ss_module* m, const double* sweep, int64_t swe
     a.items_per_grab = items_per_grab;
     a.u_layout = u_layout;
     a.pad_ = 0;
-    hipLaunchKernelGGL(zero_counter, dim3(1), dim3(64), 0, s, a.counter);
-    SS_HIP(hipGetLastError());
     void* params[] = {&a};
-    SS_HIP(launch_te(m->batch, grid_blocks, params, s, ev));
+    SS_HIP(launch_te(m->batch, grid, params, s, ev));
     return 0;
 }
 
