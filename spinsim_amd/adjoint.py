@@ -23,6 +23,7 @@ derivative of the computed forward map for every integration method.
 from __future__ import annotations
 
 import ctypes
+import re
 
 import numpy as np
 
@@ -55,14 +56,29 @@ class SsControlDesc(ctypes.Structure):
                 ("grad_offset", ctypes.c_int64)]
 
 
-def _combined_source(static, controls):
+def _leaves_q_alone(source):
+    """Whether HIP-C text plainly writes no entry 3: its subscripts are all
+    integers, and none is 3."""
+    return all(k.strip().isdigit() and int(k) != 3 for k in re.findall(r"\[([^\]]*)\]", source))
+
+
+def _combined_source(static, controls, dimension):
     """HIP-C text: the static field (renamed) plus the control terms; it sets
     SS_ADJ_CONTROLS, the adjoint kernel's number of per-lane gradient moment
-    sums, to the control count, and SS_ADJ_AXES to the set of their axes."""
+    sums, to the control count, and SS_ADJ_AXES to the set of their axes.
+
+    The backward kernel of su(2) generators fits three waves per SIMD (168
+    registers, and the LDS of up to two controls), where its table and LDS
+    latencies hide better: 2.44 -> 2.08 ms for 1024 spin-one pulses of 1e5 steps
+    on x and y.  With a quadratic shift it needs 256 registers.
+    """
     axes = 0
     for c in controls:
         axes |= 1 << c.axis
     parts = [f"#define SS_ADJ_CONTROLS {len(controls)}\n#define SS_ADJ_AXES {axes}u\n"]
+    if len(controls) <= 2 and (dimension == 2 or not axes & 8 and
+                               (static is None or _leaves_q_alone(static.source))):
+        parts.append("#define SS_ADJ_WAVES_PER_EU 3\n")
     if static is not None:
         parts.append("#define get_field ss_static_field\n" + static.source + "\n#undef get_field\n")
     call = ""
@@ -93,7 +109,7 @@ class ControlledSimulator:
             raise ValueError("the adjoint differentiates the x, y, z and q generators; "
                              "ExponentiationMethod.LIE_TROTTER_8 is not supported here")
         static = FieldSource(static_field, samplers) if static_field is not None else None
-        src = _combined_source(static, self.controls)
+        src = _combined_source(static, self.controls, spin_quantum_number.dimension)
         table_samplers = (list(static.samplers) if static is not None else []) + \
             [c.sampler for c in self.controls]
         self.n_static_tables = len(static.samplers) if static is not None else 0

@@ -1375,12 +1375,10 @@ extern "C" __device__ __attribute__((used)) char ss_module_traits[SS_PREC == 1 |
 
 // Waves per SIMD the kernels are compiled for at least: the register budget
 // is 512 / waves VGPRs a lane (in 8-register granules).  The time-evolution
-// kernels take what they need (about 230-260 for spin one: their float64
-// chains keep one or two waves per SIMD busy); the adjoint kernel is held to
-// 256, two waves per SIMD, to hide its table and LDS latencies (backward
-// pass 5.9 ms against 8.1 ms at 266 VGPRs and one wave, for 1024 spin-one
-// pulses of 1e5 steps, at the cost of a few spilled registers of its cold
-// paths).  A field source may define either to retune.
+// kernels take what they need (about 120 for spin half, 170-215 for spin one;
+// held to fewer they spill inside the step loop: 1.4 -> 2.3 ms for spin one at
+// 168).  The adjoint kernel is held to 256, two waves per SIMD, which its
+// general form needs.  A field source may define either to retune.
 #ifndef SS_WAVES_PER_EU
 #define SS_WAVES_PER_EU 1
 #endif
