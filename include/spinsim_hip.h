@@ -176,6 +176,15 @@ int ss_module_info(const ss_module *m, int *vgprs, int *sgprs, int *scratch_byte
 int ss_time_evolution(const ss_module *m, const double *sweep, double t0, double dt,
                       double dt_out, int64_t n_coarse, double *time_out, double *u_out,
                       const ss_table *tables, int lanes_per_step, ss_stream stream);
+/* evaluate() of one simulation in one call (spinsim/__init__.py:993-1085):
+ * ss_time_evolution with 1 to 32 sweep parameters given in HOST memory (they
+ * travel in the kernel arguments, so nothing is copied and the array may be
+ * reused at once), then, unless state is NULL, ss_state_scan of its operators
+ * (psi0 in host memory; spin NULL or (n, 3); workspace as there). */
+int ss_evaluate(const ss_module *m, const double *sweep, int n_sweep, double t0, double dt,
+                double dt_out, int64_t n_coarse, double *time_out, double *u_out,
+                const ss_table *tables, int lanes_per_step, const double *psi0, double *state,
+                double *spin, void *workspace, size_t workspace_bytes, ss_stream stream);
 /* Lanes per coarse step of the default launch for n_rows rows of n_fine steps
  * on `cus` compute units that hold `resident` workgroups each (host only; 1..64,
  * 1 for invalid arguments).  (No reference counterpart: a launch-planning

@@ -39,6 +39,8 @@ SIGNATURES = {
                                ctypes.POINTER(c_int), ctypes.POINTER(c_int)]),
     "ss_time_evolution": (c_int, [c_vp, c_vp, c_dbl, c_dbl, c_dbl, c_i64, c_vp, c_vp, c_vp,
                                   c_int, c_vp]),
+    "ss_evaluate": (c_int, [c_vp, c_vp, c_int, c_dbl, c_dbl, c_dbl, c_i64, c_vp, c_vp, c_vp, c_int,
+                            c_vp, c_vp, c_vp, c_vp, ctypes.c_size_t, c_vp]),
     "ss_batch_time_evolution": (c_int, [c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_vp,
                                         c_i64, c_vp, c_vp, c_vp, c_vp, c_int, c_int, c_int,
                                         c_int, c_vp]),
@@ -67,6 +69,9 @@ SIGNATURES = {
 
 # Version of the C ABI these signatures describe (ss_abi_version()).
 ABI_VERSION = 9
+
+# Sweep parameters ss_evaluate takes in the kernel arguments (SS_SWEEP_INLINE).
+SWEEP_INLINE = 32
 
 # Operator row layouts of the batch entry points (SS_U_* of the C header).
 U_FULL = 0

@@ -33,6 +33,30 @@ def batch_steps(time_start, time_end, time_step_integration, time_step_output, b
     t1 = _per_sim(time_end, b, np.float64, "time_end")
     dti = _per_sim(time_step_integration, b, np.float64, "time_step_integration")
     dto = _per_sim(time_step_output, b, np.float64, "time_step_output")
+    # evaluate()'s arithmetic on all simulations at once (round and rint are both
+    # to the nearest even)
+    with np.errstate(all="ignore"):
+        ratio = dto / dti
+        dt = dto / np.rint(np.maximum(ratio, 1))
+        rows = np.trunc((t1 - t0) / dto)
+        fine = np.floor(dto / dt + 0.5)
+        plain = (dti != 0) & (np.abs(ratio) < 2.0 ** 31) & (np.abs(rows) < 2.0 ** 62) & (fine < 2.0 ** 31)
+        warned = int((np.abs(ratio - np.rint(ratio)) > 1e-6).sum())
+    if plain.all():
+        n, nf = rows.astype(np.int64), fine.astype(np.int32)
+    else:
+        dt, n, nf, warned = _batch_steps_one_by_one(t0, t1, dti, dto, b)
+    if (n < 0).any():
+        raise ValueError("time_end is before time_start for some simulation")
+    if warned:
+        print(f"\033[33mspinsim warning!!!\n{warned} simulation(s): time_step_output not an "
+              f"integer multiple of time_step_integration; time_step_integration reset.\033[0m\n")
+    return t0, dt, dto, n, nf
+
+
+def _batch_steps_one_by_one(t0, t1, dti, dto, b):
+    """The same for steps and durations that are zero, not finite or very large, with
+    Python's errors for them."""
     dt = np.empty(b)
     n = np.empty(b, np.int64)
     nf = np.empty(b, np.int32)
@@ -44,12 +68,22 @@ def batch_steps(time_start, time_end, time_step_integration, time_step_output, b
         dt[s] = d
         n[s] = int((t1[s] - t0[s]) / d_out)
         nf[s] = math.floor(d_out / d + 0.5)
-    if (n < 0).any():
-        raise ValueError("time_end is before time_start for some simulation")
-    if warned:
-        print(f"\033[33mspinsim warning!!!\n{warned} simulation(s): time_step_output not an "
-              f"integer multiple of time_step_integration; time_step_integration reset.\033[0m\n")
-    return t0, dt, dto, n, nf
+    return dt, n, nf, warned
+
+
+def _upload(torch, device, arrays):
+    """Host arrays as device tensors, in one copy."""
+    starts, size = [], 0
+    for a in arrays:
+        starts.append(size)
+        size += -(-a.nbytes // 256) * 256
+    host = np.empty(max(size, 1), np.uint8)
+    for a, o in zip(arrays, starts):
+        host[o:o + a.nbytes] = np.ascontiguousarray(a).reshape(-1).view(np.uint8)
+    dev = torch.as_tensor(host, device=device)
+    types = {"f": torch.float64, "c": torch.complex128}
+    return [dev[o:o + a.nbytes].view(types.get(a.dtype.kind) or getattr(torch, a.dtype.name))
+            .view(a.shape) for a, o in zip(arrays, starts)]
 
 
 class BatchResults:
@@ -156,14 +190,9 @@ class BatchPlan:
         self.offsets_host = offsets
         self.fine_steps = int((n * nf.astype(np.int64)).sum())
         f64 = torch.float64
-        self.sweep = torch.as_tensor(np.ascontiguousarray(sweep), device=dev)
-        self.offsets = torch.as_tensor(offsets, device=dev)
-        self.t0 = torch.as_tensor(t0, dtype=f64, device=dev)
-        self.dt = torch.as_tensor(dt, dtype=f64, device=dev)
-        self.dt_out = torch.as_tensor(dto, dtype=f64, device=dev)
-        self.n_fine = torch.as_tensor(nf, dtype=torch.int32, device=dev)
-        self.psi0 = torch.as_tensor(np.ascontiguousarray(psi), device=dev)
-        self.counter = torch.zeros(1, dtype=torch.int64, device=dev)
+        (self.sweep, self.offsets, self.t0, self.dt, self.dt_out, self.n_fine,
+         self.psi0) = _upload(torch, dev, [sweep, offsets, t0, dt, dto, nf, psi])
+        self.counter = self.offsets  # (the launch's counter argument is not used)
         self.time = torch.empty(total, dtype=f64, device=dev)
         self.u = torch.empty((total, 2) if compact else (total, d, d), dtype=torch.complex128,
                              device=dev)
@@ -229,8 +258,9 @@ class BatchPlan:
             "ss_batch_state_scan")
 
     def run(self):
-        self.run_time_evolution()
-        self.run_state_scan()
+        stream = self.sim._torch().cuda.current_stream(self.device).cuda_stream
+        self.run_time_evolution(stream)
+        self.run_state_scan(stream)
         return self
 
     def capture(self):

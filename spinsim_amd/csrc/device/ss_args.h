@@ -3,6 +3,8 @@
 #pragma once
 
 #define SS_MAX_PHASES 8
+// Sweep parameters that travel in the kernel arguments (256 bytes).
+#define SS_SWEEP_INLINE 32
 
 // Single-simulation time-evolution launch, mirroring the reference kernel
 // get_time_evolution(sweep, time_coarse, time_end_points, dt, dt_out, U)
@@ -11,7 +13,7 @@
 // (one wave's worth of groups) covers 64 / phase_lanes[p] rows.  Items are
 // numbered phase after phase and dealt to the `waves` waves round-robin.
 struct ss_te_args {
-    const double* sweep;         // sweep_parameters (device)
+    const double* sweep;         // sweep_parameters (device), or null: sweep_inline
     const void* tables;          // ss_table[] (device) or null
     double* time_out;            // (N,) start time of each coarse step
     double* u_out;               // (N, d, d) complex128, row-major
@@ -28,6 +30,7 @@ struct ss_te_args {
     int phase_lanes[SS_MAX_PHASES];
     long long phase_row[SS_MAX_PHASES];    // first row of each phase
     long long phase_items[SS_MAX_PHASES];  // items of each phase
+    double sweep_inline[SS_SWEEP_INLINE];
 };
 
 // Batched launch: simulation s owns coarse rows [offsets[s], offsets[s+1]).

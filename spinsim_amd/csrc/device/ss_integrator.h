@@ -1386,12 +1386,27 @@ extern "C" __device__ __attribute__((used)) char ss_module_traits[SS_PREC == 1 |
 #define SS_ADJ_WAVES_PER_EU 2
 #endif
 #define SS_KERNEL_ATTR __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SS_WAVES_PER_EU)))
+// The sweep parameters of a single-simulation launch: its device array, or the
+// values in the kernel arguments (read where they lie, in the kernarg segment;
+// a host call then copies nothing: 15 us less).
+static __device__ __forceinline__ const double* ss_te_sweep(const ss_te_args& a)
+{
+    // (both as global addresses: with a flat one the callback's loads stay in the
+    // step loop, 215 -> 270 us for the noisy run's 24 parameters)
+    typedef const __attribute__((address_space(1))) double* global_ptr;
+    global_ptr p = (global_ptr)a.sweep;
+    if (!p)
+        p = (global_ptr)((unsigned long long)__builtin_amdgcn_kernarg_segment_ptr() +
+                         __builtin_offsetof(ss_te_args, sweep_inline));
+    return (const double*)p;
+}
+
 // One item of a single-simulation launch (get_time_evolution,
 // spinsim/__init__.py:854-896): in phase p, whose items start at item number
 // `first`, group gi of `lanes` lanes integrates coarse row
 // phase_row[p] + (item - first) * (64 / lanes) + gi.
-static __device__ __forceinline__ void ss_te_item(const ss_te_args& a, long long item, int p, long long first,
-                                                  const ss_ctx* ctx)
+static __device__ __forceinline__ void ss_te_item(const ss_te_args& a, const double* sweep, long long item, int p,
+                                                  long long first, const ss_ctx* ctx)
 {
     const int lane = threadIdx.x & 63;
     const int lanes = a.phase_lanes[p];
@@ -1406,9 +1421,9 @@ static __device__ __forceinline__ void ss_te_item(const ss_te_args& a, long long
     const int j0 = rank * base + (rank < rem ? rank : rem);
     const int count = active ? base + (rank < rem ? 1 : 0) : 0;
     const double tc = ss_coarse_time(a.t0, a.dt_out, row);
-    const double rot = active ? ss_rotating_wave(tc, a.dt_out, a.sweep, ctx) : 0.0;
+    const double rot = active ? ss_rotating_wave(tc, a.dt_out, sweep, ctx) : 0.0;
     ss_cd u[SS_D][SS_D];
-    ss_integrate(u, j0, count, tc, rot, a.dt, a.off_a, a.off_b, a.sweep, ctx);
+    ss_integrate(u, j0, count, tc, rot, a.dt, a.off_a, a.off_b, sweep, ctx);
     ss_group_reduce(u, rank, lanes);
     if (active && rank == 0) ss_store(u, rot, a.dt_out, tc, row, a.time_out, a.u_out);
 }
@@ -1423,7 +1438,7 @@ extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_kernel(ss_te_args a)
     ss_ctx ctx;
     ctx.tables = reinterpret_cast<const ss_table*>(a.tables);
     ctx.sim = 0;
-    ss_te_item(a, wave, 0, 0, &ctx);
+    ss_te_item(a, ss_te_sweep(a), wave, 0, 0, &ctx);
 }
 
 // One simulation on a given number of waves: wave w takes items w, w + waves,
@@ -1437,6 +1452,7 @@ extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_phased_kernel(ss_te_
     ss_ctx ctx;
     ctx.tables = reinterpret_cast<const ss_table*>(a.tables);
     ctx.sim = 0;
+    const double* sweep = ss_te_sweep(a);
 #pragma unroll 1
     for (long long item = wave; item < a.items; item += a.waves) {
         int p = 0;
@@ -1445,7 +1461,7 @@ extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_phased_kernel(ss_te_
             first += a.phase_items[p];
             ++p;
         }
-        ss_te_item(a, item, p, first, &ctx);
+        ss_te_item(a, sweep, item, p, first, &ctx);
     }
 }
 

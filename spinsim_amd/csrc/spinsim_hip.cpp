@@ -1475,25 +1475,27 @@ int ss_time_evolution_plan(int64_t n_coarse, int n_fine, int64_t waves, int* n_p
     return 0;
 }
 
-int ss_time_evolution(const ss_module* m, const double* sweep, double t0, double dt, double dt_out,
-                      int64_t n_coarse, double* time_out, double* u_out, const ss_table* tables,
-                      int lanes_per_step, ss_stream stream)
+// ss_time_evolution with the sweep parameters in a device array, or (sweep null)
+// n_inline of them in host memory, which go into the kernel arguments.
+static int time_evolution(const char* who, const ss_module* m, const double* sweep, const double* sweep_host,
+                          int n_inline, double t0, double dt, double dt_out, int64_t n_coarse, double* time_out,
+                          double* u_out, const ss_table* tables, int lanes_per_step, ss_stream stream)
 {
     const TeEvents ev = take_te_events();
-    if (!m) return fail("ss_time_evolution: null module");
-    if (n_coarse < 0) return fail("ss_time_evolution: negative n_coarse");
+    if (!m) return fail("%s: null module", who);
+    if (n_coarse < 0) return fail("%s: negative n_coarse", who);
     if (n_coarse == 0) return 0;
-    if (!sweep || !time_out || !u_out) return fail("ss_time_evolution: null buffer");
-    if (!(dt > 0) || !(dt_out > 0)) return fail("ss_time_evolution: steps must be positive");
+    if ((!sweep && !sweep_host) || !time_out || !u_out) return fail("%s: null buffer", who);
+    if (!(dt > 0) || !(dt_out > 0)) return fail("%s: steps must be positive", who);
     const double nf = std::floor(dt_out / dt + 0.5);  // :832
-    if (!(nf >= 0) || nf > 2147483647.0) return fail("ss_time_evolution: bad fine-step count");
+    if (!(nf >= 0) || nf > 2147483647.0) return fail("%s: bad fine-step count", who);
     const int n_fine = int(nf);
-    if (lanes_per_step > 64 || lanes_per_step < -64)
-        return fail("ss_time_evolution: lanes_per_step must be in -64..64");
-    if (n_coarse > (1LL << 40)) return fail("ss_time_evolution: n_coarse too large");
+    if (lanes_per_step > 64 || lanes_per_step < -64) return fail("%s: lanes_per_step must be in -64..64", who);
+    if (n_coarse > (1LL << 40)) return fail("%s: n_coarse too large", who);
     ss_te_args a;
     std::memset(&a, 0, sizeof(a));
     a.sweep = sweep;
+    if (!sweep) std::memcpy(a.sweep_inline, sweep_host, size_t(n_inline) * sizeof(double));
     a.tables = tables;
     a.time_out = time_out;
     a.u_out = u_out;
@@ -1517,10 +1519,34 @@ int ss_time_evolution(const ss_module* m, const double* sweep, double t0, double
         plan_phases(n_coarse, n_fine, (long long)(-lanes_per_step) * m->cus * 4, &a);
     }
     const long long blocks = (a.waves + 3) / 4;
-    if (blocks > 2147483647LL) return fail("ss_time_evolution: grid too large");
+    if (blocks > 2147483647LL) return fail("%s: grid too large", who);
     void* params[] = {&a};
     SS_HIP(launch_te(lanes_per_step > 0 ? m->single : m->phased, blocks, params, static_cast<hipStream_t>(stream), ev));
     return 0;
+}
+
+int ss_time_evolution(const ss_module* m, const double* sweep, double t0, double dt, double dt_out,
+                      int64_t n_coarse, double* time_out, double* u_out, const ss_table* tables,
+                      int lanes_per_step, ss_stream stream)
+{
+    return time_evolution("ss_time_evolution", m, sweep, nullptr, 0, t0, dt, dt_out, n_coarse, time_out, u_out, tables,
+                          lanes_per_step, stream);
+}
+
+int ss_evaluate(const ss_module* m, const double* sweep, int n_sweep, double t0, double dt, double dt_out,
+                int64_t n_coarse, double* time_out, double* u_out, const ss_table* tables, int lanes_per_step,
+                const double* psi0, double* state, double* spin, void* workspace, size_t workspace_bytes,
+                ss_stream stream)
+{
+    if (n_sweep < 1 || n_sweep > SS_SWEEP_INLINE) {
+        (void)take_te_events();
+        return fail("ss_evaluate: 1 to %d sweep parameters, got %d", SS_SWEEP_INLINE, n_sweep);
+    }
+    if (int rc = time_evolution("ss_evaluate", m, nullptr, sweep, n_sweep, t0, dt, dt_out, n_coarse, time_out, u_out,
+                                tables, lanes_per_step, stream))
+        return rc;
+    if (!state) return 0;
+    return ss_state_scan(psi0, u_out, state, spin, n_coarse, m->dim, workspace, workspace_bytes, stream);
 }
 
 int ss_batch_time_evolution(const ss_module* m, const double* sweep, int64_t sweep_stride, int64_t n_sims,

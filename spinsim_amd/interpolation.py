@@ -66,6 +66,7 @@ class InterpolationSampler:
         self.zero_boundary = bool(zero_boundary)
         self.version = 0
         self._device = {}
+        self._device_time = {}
         self._bound = None
 
     @property
@@ -104,33 +105,46 @@ class InterpolationSampler:
         """Read the amplitudes from a device tensor view: row s of the table starts
         at ``amplitude_rows.data_ptr() + s*stride`` doubles (no copy).  Used for
         differentiable control amplitudes."""
-        self._bound = (amplitude_rows, int(stride))
-        self.version += 1
+        old, self._bound = self._bound, (amplitude_rows, int(stride))
+        # (a table holds the rows' address and stride: rows bound at the same ones
+        # need no new table)
+        if old is None or (old[0].data_ptr(), old[0].device, old[1]) != (
+                amplitude_rows.data_ptr(), amplitude_rows.device, int(stride)):
+            self.version += 1
 
     def unbind(self):
         self._bound = None
         self.version += 1
 
-    def device_arrays(self, device):
-        """(time, amplitude) as float64 tensors on ``device`` (cached)."""
+    def _time_on(self, device):
+        """The time grid as a float64 tensor on ``device`` (it never changes)."""
         import torch
 
+        key = str(device)
+        if key not in self._device_time:
+            self._device_time[key] = torch.as_tensor(self.time, device=device)
+        return self._device_time[key]
+
+    def device_arrays(self, device):
+        """(time, amplitude) as float64 tensors on ``device`` (cached): the bound
+        rows where amplitudes are bound."""
+        import torch
+
+        if self._bound is not None:
+            return self._time_on(device), self._bound[0]
         key = (str(device), self.version)
         if key not in self._device:
             self._device.clear()
-            t = torch.as_tensor(self.time, device=device)
             a = torch.as_tensor(self.amplitude, device=device).contiguous()
-            self._device[key] = (t, a)
+            self._device[key] = (self._time_on(device), a)
         return self._device[key]
 
     def table_record(self, device) -> SsTable:
         t, a = self.device_arrays(device)
         rec = SsTable()
         self._fill(rec, t.data_ptr(), a.data_ptr())
-        bound = getattr(self, "_bound", None)
-        if bound is not None:
-            rec.amplitude = bound[0].data_ptr()
-            rec.amplitude_stride = bound[1]
+        if self._bound is not None:
+            rec.amplitude_stride = self._bound[1]
         return rec
 
     def host_record(self):

@@ -122,6 +122,9 @@ class FieldSource:
 # Largest evaluate() result (time, U and state) staged through pinned host
 # memory; larger results are copied to pageable memory directly.
 PINNED_RESULT_BYTES = 1 << 31
+# Largest one (with its Bloch vectors) that is computed into one device buffer and
+# comes back in one copy; below, a copy's latency outweighs its bytes.
+SINGLE_COPY_BYTES = 1 << 20
 
 
 class Results:
@@ -133,23 +136,39 @@ class Results:
     tensors.
     """
 
-    def __init__(self, time, time_evolution, state, spin_calculator, _device_state=None):
+    def __init__(self, time, time_evolution, state, spin_calculator, _device_state=None,
+                 _spin=None):
         self.time = time
         self.time_evolution = time_evolution
         self.state = state
         self.spin_calculator = spin_calculator
         self._device_state = _device_state
+        self._spin = _spin
 
     def __getattr__(self, attr_name: str):
         if attr_name == "spin":
             src = self.__dict__.get("_device_state")
-            if src is not None and isinstance(self.__dict__["state"], np.ndarray):
-                spin = self.spin_calculator(src).cpu().numpy()
+            if self.__dict__.get("_spin") is not None:
+                spin = self.__dict__["_spin"]
+            elif src is not None and isinstance(self.__dict__["state"], np.ndarray):
+                spin = _to_numpy(self.spin_calculator(src))
             else:
                 spin = self.spin_calculator(self.__dict__["state"])
             setattr(self, attr_name, spin)
             return spin
         raise AttributeError("{} has no attribute called {}.".format(self, attr_name))
+
+
+def _to_numpy(tensor):
+    """A device tensor as a numpy array, through pinned memory up to the limit
+    (a copy to pageable memory goes through staging buffers)."""
+    import torch
+    if tensor.numel() * tensor.element_size() > PINNED_RESULT_BYTES:
+        return tensor.cpu().numpy()
+    host = torch.empty(tensor.shape, dtype=tensor.dtype, pin_memory=True)
+    host.copy_(tensor, non_blocking=True)
+    torch.cuda.current_stream(tensor.device).synchronize()
+    return host.numpy()
 
 
 def _default_device():
@@ -391,19 +410,20 @@ class Simulator:
         u_out (N, d, d) complex128 are contiguous device tensors."""
         torch = self._torch()
         dev = u_out.device
-        n = int(time_out.shape[0])
         lanes = lanes_per_step if lanes_per_step is not None else (self.lanes_per_step or 0)
+        if stream is None:
+            stream = torch.cuda.current_stream(dev).cuda_stream
+        self._launch_time_evolution(sweep, t0, dt, dt_out, int(time_out.shape[0]), dev,
+                                    time_out.data_ptr(), u_out.data_ptr(), lanes, stream)
+
+    def _launch_time_evolution(self, sweep, t0, dt, dt_out, n, dev, time_ptr, u_ptr, lanes, stream):
         if lanes == "auto":
             from .autotune import tune_lanes
             n_fine = math.floor(dt_out / dt + 0.5)
             lanes, _ = tune_lanes(self, n, n_fine, dt, dt_out, sweep, t0) if n else (0, None)
-        if stream is None:
-            stream = torch.cuda.current_stream(dev).cuda_stream
-        mod = self._module(dev)
         _native.check(_native.lib().ss_time_evolution(
-            mod.handle, sweep.data_ptr(), float(t0), float(dt), float(dt_out), n,
-            time_out.data_ptr(), u_out.data_ptr(), self._table_ptr(dev), int(lanes), stream),
-            "ss_time_evolution")
+            self._module(dev).handle, sweep.data_ptr(), float(t0), float(dt), float(dt_out), n,
+            time_ptr, u_ptr, self._table_ptr(dev), int(lanes), stream), "ss_time_evolution")
 
     def launch_state_scan(self, psi0, u, state, workspace, spin=None, stream=None):
         """Enqueue ss_state_scan (and the Bloch vectors into ``spin`` when given);
@@ -513,33 +533,79 @@ class Simulator:
         dt, n, ends = derive_steps(time_start, time_end, time_step_integration, time_step_output)
         if n < 0:
             raise ValueError("time_end is before time_start")
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("evaluate() cannot be captured in a graph: launch into buffers of "
+                               "your own, or capture a BatchPlan")
         d = self.dimension
         dev = torch.device("cuda", torch.cuda.current_device())
+        stream = torch.cuda.current_stream(dev)
+        sweep = np.ascontiguousarray(np.atleast_1d(np.asarray(sweep_parameters, np.float64)))
+        lanes = lanes_per_step if lanes_per_step is not None else (self.lanes_per_step or 0)
+        if not 1 <= sweep.size <= _native.SWEEP_INLINE or lanes == "auto":
+            sweep = torch.as_tensor(sweep, device=dev)
+        psi0 = np.ascontiguousarray(np.asarray(state_init, np.complex128).reshape(d))
+        ws_bytes = int(_native.lib().ss_state_scan_workspace(n, d))
+
+        def run(time, u, state, spin, ws):
+            """Enqueue time evolution and, with a state, the scan (device addresses)."""
+            if isinstance(sweep, np.ndarray):
+                _native.check(_native.lib().ss_evaluate(
+                    self._module(dev).handle, sweep.ctypes.data, sweep.size, float(ends[0]), dt,
+                    float(time_step_output), n, time, u, self._table_ptr(dev), int(lanes),
+                    psi0.ctypes.data, state, spin, ws, ws_bytes, stream.cuda_stream),
+                    "ss_evaluate")
+                return
+            self._launch_time_evolution(sweep, float(ends[0]), dt, time_step_output, n, dev, time,
+                                        u, lanes, stream.cuda_stream)
+            if state:
+                _native.check(_native.lib().ss_state_scan(
+                    psi0.ctypes.data, u, state, spin, n, d, ws, ws_bytes, stream.cuda_stream),
+                    "ss_state_scan")
+
+        # time, U, state and spin one after the other, 256-byte aligned, for
+        # results that come back in one copy
+        shapes = (((n,), 8), ((n, d, d), 16), ((n, d), 16), ((n, 3), 8))
+        starts, size = [], 0
+        for shape, item in shapes:
+            starts.append(size)
+            size += -(-math.prod(shape) * item // 256) * 256
+        if output == "numpy" and size <= min(SINGLE_COPY_BYTES, PINNED_RESULT_BYTES):
+            buf = torch.empty(size + max(ws_bytes, 1), dtype=torch.uint8, device=dev)
+            base = buf.data_ptr()
+            run(*(base + o for o in starts), base + size)
+            host = torch.empty(size, dtype=torch.uint8, pin_memory=True)
+            host.copy_(buf[:size], non_blocking=True)
+            stream.synchronize()
+            host = host.numpy()
+            time, u, state, spin = (
+                host[o:o + math.prod(shape) * item].view(np.complex128 if item == 16 else np.float64)
+                .reshape(shape) for o, (shape, item) in zip(starts, shapes))
+            return Results(time, u, state, self.spin_calculator, _spin=spin)
         time = torch.empty(n, dtype=torch.float64, device=dev)
         u = torch.empty((n, d, d), dtype=torch.complex128, device=dev)
-        self._get_time_evolution(sweep_parameters, time, ends, dt, time_step_output, u,
-                                 lanes_per_step=lanes_per_step)
+        state = torch.empty((n, d), dtype=torch.complex128, device=dev)
+        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
         if output == "torch":
-            return Results(time, u, self.state_scan(state_init, u), self.spin_calculator)
-        # numpy results: time and U go to pinned host memory on a side stream
-        # while the state scan runs, then the states follow
-        pinned = n * (d * d + d + 1) * 16 <= PINNED_RESULT_BYTES
-        if not pinned:
-            state = self.state_scan(state_init, u)
+            run(time.data_ptr(), u.data_ptr(), state.data_ptr(), None, ws.data_ptr())
+            return Results(time, u, state, self.spin_calculator)
+        # larger numpy results: time and U go to pinned host memory on a side
+        # stream while the state scan runs, then the states follow
+        if n * (d * d + d + 1) * 16 > PINNED_RESULT_BYTES:
+            run(time.data_ptr(), u.data_ptr(), state.data_ptr(), None, ws.data_ptr())
             return Results(time.cpu().numpy(), u.cpu().numpy(), state.cpu().numpy(),
                            self.spin_calculator, _device_state=state)
-        main = torch.cuda.current_stream(dev)
         side = self._copy_stream(dev)
         h_time = torch.empty(time.shape, dtype=time.dtype, pin_memory=True)
         h_u = torch.empty(u.shape, dtype=u.dtype, pin_memory=True)
         h_state = torch.empty((n, d), dtype=u.dtype, pin_memory=True)
-        side.wait_stream(main)
+        run(time.data_ptr(), u.data_ptr(), None, None, None)
+        side.wait_stream(stream)
         with torch.cuda.stream(side):
             h_time.copy_(time, non_blocking=True)
             h_u.copy_(u, non_blocking=True)
-        state = self.state_scan(state_init, u)
+        self.launch_state_scan(psi0, u, state, ws, stream=stream.cuda_stream)
         h_state.copy_(state, non_blocking=True)
-        main.synchronize()
+        stream.synchronize()
         side.synchronize()
         return Results(h_time.numpy(), h_u.numpy(), h_state.numpy(), self.spin_calculator,
                        _device_state=state)
