@@ -920,11 +920,22 @@ static __device__ __forceinline__ void ss_gen_dense(const ss_gen& a, ss_cf m[SS_
 // cos(theta) I + (sin(theta)/theta) A and the residual is exactly
 // B = (cos theta - 1) I + (sin theta / theta - 1) A.  The two scalars come from
 // their Taylor series in theta^2 (to theta^10; truncation below 1e-11 relative
-// for theta <= 1/2) in float32, or from float64 sincos beyond.
+// for theta <= 1/2) in float32, or from float64 sincos beyond.  Up to theta =
+// 3e-3 two terms of each do: the third is below 3e-13 of them, which changes
+// their float32 rounding in about one step of 2e5 (4096 spin-half runs: 13.18 ->
+// 12.98 ms, the same bits).
+#define SS_RESIDUAL_SHORT 1e-5
 static __device__ __forceinline__ void ss_expo_residual(const double* g, ss_cf b[SS_D][SS_D])
 {
     const double th2 = 0.25 * (g[0] * g[0] + g[1] * g[1] + g[2] * g[2]);
     ss_bulk c1, c2;
+#if SS_PREC != 2
+    if (th2 <= SS_RESIDUAL_SHORT) {
+        const ss_bulk t2 = (ss_bulk)th2;
+        c1 = t2 * SS_BULK_FMA(t2, (ss_bulk)4.1666666666666664e-02, (ss_bulk)-0.5);
+        c2 = t2 * SS_BULK_FMA(t2, (ss_bulk)8.333333333333333e-03, (ss_bulk)-0.16666666666666666);
+    } else
+#endif
     if (th2 <= 0.25) {
         const ss_bulk t2 = (ss_bulk)th2;
         c1 = t2 * SS_BULK_FMA(t2, SS_BULK_FMA(t2, SS_BULK_FMA(t2, SS_BULK_FMA(t2, (ss_bulk)-2.7557319223985893e-07,
