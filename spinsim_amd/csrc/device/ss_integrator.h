@@ -1444,6 +1444,7 @@ static __device__ __forceinline__ void ss_te_item(const ss_te_args& a, const dou
 extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_kernel(ss_te_args a)
 {
     ss_trig_load();
+    ss_exp_load();
     const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     if (wave >= a.items) return;  // whole waves only
     ss_ctx ctx;
@@ -1459,6 +1460,7 @@ extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_kernel(ss_te_args a)
 extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_phased_kernel(ss_te_args a)
 {
     ss_trig_load();
+    ss_exp_load();
     const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     ss_ctx ctx;
     ctx.tables = reinterpret_cast<const ss_table*>(a.tables);
@@ -1486,6 +1488,7 @@ extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_phased_kernel(ss_te_
 extern "C" __global__ void SS_KERNEL_ATTR ss_batch_time_evolution_kernel(ss_batch_args a)
 {
     ss_trig_load();
+    ss_exp_load();
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lanes = a.lanes_per_step;
@@ -2079,6 +2082,7 @@ ss_batch_adjoint_kernel(ss_adjoint_args a)
     // accesses to one slot are consecutive doubles, free of LDS bank conflicts
     extern __shared__ double ss_adj_windows[];
     ss_trig_load();
+    ss_exp_load();
     const long long row = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     double* win = ss_adj_windows + threadIdx.x;
 #pragma unroll

@@ -1147,9 +1147,11 @@ std::string build_source(const char* field_src, int dim, int method, int expo, i
     // the windings of each coarse step read it; and where the adjoint kernel is
     // specialised for its controls, the 16 KiB would halve its workgroups at
     // three controls.
-    const bool lds = (std::strstr(field_src, "cos") || std::strstr(field_src, "sin")) &&
-                     !std::strstr(field_src, "SS_ADJ_AXES");
-    if (lds) s += "#define SS_TRIG_LDS 1\n";
+    // The table of exp likewise (2 KiB).
+    if (!std::strstr(field_src, "SS_ADJ_AXES")) {
+        if (std::strstr(field_src, "cos") || std::strstr(field_src, "sin")) s += "#define SS_TRIG_LDS 1\n";
+        if (std::strstr(field_src, "exp")) s += "#define SS_EXP_LDS 1\n";
+    }
     char head[512];
     snprintf(head, sizeof(head),
              "#define SS_DIM %d\n#define SS_LIE %d\n#define SS_METHOD %d\n#define SS_EXPO %d\n"
