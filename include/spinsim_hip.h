@@ -180,11 +180,15 @@ int ss_time_evolution(const ss_module *m, const double *sweep, double t0, double
  * ss_time_evolution with 1 to 32 sweep parameters given in HOST memory (they
  * travel in the kernel arguments, so nothing is copied and the array may be
  * reused at once), then, unless state is NULL, ss_state_scan of its operators
- * (psi0 in host memory; spin NULL or (n, 3); workspace as there). */
+ * (psi0 in host memory; spin NULL or (n, 3); a workspace of that call's size).
+ * With a workspace of ss_evaluate_workspace bytes the integrator leaves the
+ * scan's products itself where its launch has at most 1024 workgroups, and one
+ * pass writes the states. */
 int ss_evaluate(const ss_module *m, const double *sweep, int n_sweep, double t0, double dt,
                 double dt_out, int64_t n_coarse, double *time_out, double *u_out,
                 const ss_table *tables, int lanes_per_step, const double *psi0, double *state,
                 double *spin, void *workspace, size_t workspace_bytes, ss_stream stream);
+size_t ss_evaluate_workspace(int64_t n, int dim);
 /* Lanes per coarse step of the default launch for n_rows rows of n_fine steps
  * on `cus` compute units that hold `resident` workgroups each (host only; 1..64,
  * 1 for invalid arguments).  (No reference counterpart: a launch-planning

@@ -30,6 +30,8 @@ struct ss_te_args {
     int phase_lanes[SS_MAX_PHASES];
     long long phase_row[SS_MAX_PHASES];    // first row of each phase
     long long phase_items[SS_MAX_PHASES];  // items of each phase
+    double* prefix;              // (N, d, d) with block_total: the operators' products (ss_scan_block); or null
+    double* block_total;         // (workgroups, d, d)
     double sweep_inline[SS_SWEEP_INLINE];
 };
 

@@ -301,17 +301,12 @@ __global__ void __launch_bounds__(kSingleScanBlock) single_scan_apply(const doub
     }
 }
 
-// Single simulation with at most kFusedScanBlocks blocks, passes 2 and 3 in one:
-// each workgroup forms its own carry-in state, v_b = (T_{b-1} ... T_0) psi0,
-// from the block totals (up to four consecutive ones per thread, an ordered
-// shuffle tree per wave, the four wave products through LDS), then applies it
-// like single_scan_apply.
+// Carry-in state of this workgroup, v_b = (T_{b-1} ... T_0) psi0, from the
+// totals before it: consecutive ones per thread, an ordered shuffle tree per
+// wave, the four wave products through LDS.  Each workgroup forms its own, so
+// no pass of one workgroup stands between the totals and the states.
 template <int D>
-__global__ void __launch_bounds__(kSingleScanBlock) single_scan_apply_carry(const double* u, long long n,
-                                                                 const double* lane_prefix,
-                                                                 const double* block_total, ss_cd p0,
-                                                                 ss_cd p1, ss_cd p2, double* state,
-                                                                 double* spin)
+__device__ __forceinline__ void block_carry(const double* block_total, ss_cd p0, ss_cd p1, ss_cd p2, ss_cd c[D])
 {
     __shared__ ss_cd wave_prod[kSingleScanBlock / 64][D][D];
     __shared__ ss_cd carry[D];
@@ -324,9 +319,10 @@ __global__ void __launch_bounds__(kSingleScanBlock) single_scan_apply_carry(cons
         load_mat<D>(block_total, b, tot);
         ss_left_multiply<D>(tot, m);
     }
-    // product over the wave's lanes, later totals on the left
+    // product over the wave's lanes, later totals on the left (lanes from the
+    // workgroup's number on hold the identity)
 #pragma unroll 1
-    for (int s = 1; s < 64; s <<= 1) {
+    for (int s = 1; s < 64 && s < (int)blockIdx.x; s <<= 1) {
         ss_cd o[D][D];
         shfl_down_mat<D>(m, o, s);
         if ((lane & (2 * s - 1)) == 0) ss_left_multiply<D>(o, m);
@@ -336,7 +332,8 @@ __global__ void __launch_bounds__(kSingleScanBlock) single_scan_apply_carry(cons
     if (t == 0) {
         ss_cd pr[D][D];
         ss_copy<D>(wave_prod[0], pr);
-        for (int w = 1; w < kSingleScanBlock / 64; ++w) ss_left_multiply<D>(wave_prod[w], pr);
+        for (int w = 1; w < kSingleScanBlock / 64 && 64 * w * per < (int)blockIdx.x; ++w)
+            ss_left_multiply<D>(wave_prod[w], pr);
         const ss_cd psi[3] = {p0, p1, p2};
         ss_cd v[D];
         ss_matvec<D>(pr, psi, v);
@@ -344,14 +341,27 @@ __global__ void __launch_bounds__(kSingleScanBlock) single_scan_apply_carry(cons
         for (int r = 0; r < D; ++r) carry[r] = v[r];
     }
     __syncthreads();
-    const long long lane_id = (long long)blockIdx.x * kSingleScanBlock + t;
+#pragma unroll
+    for (int r = 0; r < D; ++r) c[r] = carry[r];
+}
+
+// Single simulation with at most kFusedScanBlocks blocks, passes 2 and 3 in one:
+// block_carry, then the states like single_scan_apply.
+template <int D>
+__global__ void __launch_bounds__(kSingleScanBlock) single_scan_apply_carry(const double* u, long long n,
+                                                                 const double* lane_prefix,
+                                                                 const double* block_total, ss_cd p0,
+                                                                 ss_cd p1, ss_cd p2, double* state,
+                                                                 double* spin)
+{
+    ss_cd c[D];
+    block_carry<D>(block_total, p0, p1, p2, c);
+    const long long lane_id = (long long)blockIdx.x * kSingleScanBlock + threadIdx.x;
     const long long k0 = lane_id * kSingleScanChunk;
     if (k0 >= n) return;
     const long long kend = k0 + kSingleScanChunk < n ? k0 + kSingleScanChunk : n;
-    ss_cd pre[D][D], c[D], v[D];
+    ss_cd pre[D][D], v[D];
     load_mat<D>(lane_prefix, lane_id, pre);
-#pragma unroll
-    for (int r = 0; r < D; ++r) c[r] = carry[r];
     ss_matvec<D>(pre, c, v);
     for (long long k = k0; k < kend; ++k) {
         store_vec<D>(state, k, v);
@@ -364,6 +374,25 @@ __global__ void __launch_bounds__(kSingleScanBlock) single_scan_apply_carry(cons
             for (int r = 0; r < D; ++r) v[r] = tv[r];
         }
     }
+}
+
+// The states of a time evolution that left its products (ss_scan_block of the
+// integrator): workgroup b holds rows [rows * b, rows * b + rows), and
+// state[k] = prefix[k] v_b.
+template <int D>
+__global__ void __launch_bounds__(kSingleScanBlock) evaluate_states(const double* prefix, long long n, int rows,
+                                                         const double* block_total, ss_cd p0, ss_cd p1,
+                                                         ss_cd p2, double* state, double* spin)
+{
+    const long long k = (long long)blockIdx.x * rows + threadIdx.x;
+    const bool active = (int)threadIdx.x < rows && k < n;
+    ss_cd pre[D][D], c[D], v[D];
+    if (active) load_mat<D>(prefix, k, pre);
+    block_carry<D>(block_total, p0, p1, p2, c);
+    if (!active) return;
+    ss_matvec<D>(pre, c, v);
+    store_vec<D>(state, k, v);
+    if (spin) ss_store_spin<D>(v, spin, k);
 }
 
 // ---- state scan: get_state (:1087-1111) batches and costates, two passes -----
@@ -1108,6 +1137,13 @@ SingleScanLayout single_scan_layout(int64_t n, int dim)
     return l;
 }
 
+// Workspace of ss_evaluate's scan: a product per row, a total per workgroup.
+size_t evaluate_total_off(int64_t n, int dim) { return align256(size_t(n) * dim * dim * 16); }
+size_t evaluate_bytes(int64_t n, int dim)
+{
+    return evaluate_total_off(n, dim) + align256(size_t(kFusedScanBlocks) * dim * dim * 16);
+}
+
 struct ScanLayout {
     long long tiles, chunk_rows, chunks;
     size_t bytes;
@@ -1488,11 +1524,21 @@ int ss_time_evolution_plan(int64_t n_coarse, int n_fine, int64_t waves, int* n_p
     return 0;
 }
 
+// Where a time evolution may leave its operators' products (workspace of
+// evaluate_bytes), and what it left: the launch's workgroups, 0 for no products,
+// and the rows of each.
+struct EvaluateScan {
+    double *prefix, *block_total;
+    long long blocks;
+    int rows;
+};
+
 // ss_time_evolution with the sweep parameters in a device array, or (sweep null)
 // n_inline of them in host memory, which go into the kernel arguments.
 static int time_evolution(const char* who, const ss_module* m, const double* sweep, const double* sweep_host,
                           int n_inline, double t0, double dt, double dt_out, int64_t n_coarse, double* time_out,
-                          double* u_out, const ss_table* tables, int lanes_per_step, ss_stream stream)
+                          double* u_out, const ss_table* tables, int lanes_per_step, EvaluateScan* scan,
+                          ss_stream stream)
 {
     const TeEvents ev = take_te_events();
     if (!m) return fail("%s: null module", who);
@@ -1533,6 +1579,12 @@ static int time_evolution(const char* who, const ss_module* m, const double* swe
     }
     const long long blocks = (a.waves + 3) / 4;
     if (blocks > 2147483647LL) return fail("%s: grid too large", who);
+    if (scan && lanes_per_step > 0 && blocks <= kFusedScanBlocks) {
+        a.prefix = scan->prefix;
+        a.block_total = scan->block_total;
+        scan->blocks = blocks;
+        scan->rows = 4 * (64 / lanes_per_step);
+    }
     void* params[] = {&a};
     SS_HIP(launch_te(lanes_per_step > 0 ? m->single : m->phased, blocks, params, static_cast<hipStream_t>(stream), ev));
     return 0;
@@ -1543,7 +1595,14 @@ int ss_time_evolution(const ss_module* m, const double* sweep, double t0, double
                       int lanes_per_step, ss_stream stream)
 {
     return time_evolution("ss_time_evolution", m, sweep, nullptr, 0, t0, dt, dt_out, n_coarse, time_out, u_out, tables,
-                          lanes_per_step, stream);
+                          lanes_per_step, nullptr, stream);
+}
+
+size_t ss_evaluate_workspace(int64_t n, int dim)
+{
+    if (n <= 0 || (dim != 2 && dim != 3)) return 0;
+    const size_t scan = ss_state_scan_workspace(n, dim);
+    return n <= kFusedScanBlocks * 256LL ? std::max(scan, evaluate_bytes(n, dim)) : scan;
 }
 
 int ss_evaluate(const ss_module* m, const double* sweep, int n_sweep, double t0, double dt, double dt_out,
@@ -1555,11 +1614,30 @@ int ss_evaluate(const ss_module* m, const double* sweep, int n_sweep, double t0,
         (void)take_te_events();
         return fail("ss_evaluate: 1 to %d sweep parameters, got %d", SS_SWEEP_INLINE, n_sweep);
     }
+    // up to kFusedScanBlocks workgroups the integrator does the scan's first pass
+    EvaluateScan scan = {};
+    if (m && psi0 && state && workspace && n_coarse > 0 && n_coarse <= kFusedScanBlocks * 256LL &&
+        workspace_bytes >= evaluate_bytes(n_coarse, m->dim)) {
+        scan.prefix = static_cast<double*>(workspace);
+        scan.block_total = reinterpret_cast<double*>(static_cast<char*>(workspace) + evaluate_total_off(n_coarse, m->dim));
+    }
     if (int rc = time_evolution("ss_evaluate", m, nullptr, sweep, n_sweep, t0, dt, dt_out, n_coarse, time_out, u_out,
-                                tables, lanes_per_step, stream))
+                                tables, lanes_per_step, scan.prefix ? &scan : nullptr, stream))
         return rc;
     if (!state) return 0;
-    return ss_state_scan(psi0, u_out, state, spin, n_coarse, m->dim, workspace, workspace_bytes, stream);
+    if (!scan.blocks) return ss_state_scan(psi0, u_out, state, spin, n_coarse, m->dim, workspace, workspace_bytes, stream);
+    const ss_cd p0 = ss_c(psi0[0], psi0[1]), p1 = ss_c(psi0[2], psi0[3]);
+    const ss_cd p2 = m->dim == 3 ? ss_c(psi0[4], psi0[5]) : ss_c(0, 0);
+    const dim3 grid(unsigned(scan.blocks)), block(kSingleScanBlock);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (m->dim == 2)
+        hipLaunchKernelGGL(evaluate_states<2>, grid, block, 0, s, scan.prefix, (long long)n_coarse, scan.rows,
+                           scan.block_total, p0, p1, p2, state, spin);
+    else
+        hipLaunchKernelGGL(evaluate_states<3>, grid, block, 0, s, scan.prefix, (long long)n_coarse, scan.rows,
+                           scan.block_total, p0, p1, p2, state, spin);
+    SS_HIP(hipGetLastError());
+    return 0;
 }
 
 int ss_batch_time_evolution(const ss_module* m, const double* sweep, int64_t sweep_stride, int64_t n_sims,

@@ -544,7 +544,7 @@ class Simulator:
         if not 1 <= sweep.size <= _native.SWEEP_INLINE or lanes == "auto":
             sweep = torch.as_tensor(sweep, device=dev)
         psi0 = np.ascontiguousarray(np.asarray(state_init, np.complex128).reshape(d))
-        ws_bytes = int(_native.lib().ss_state_scan_workspace(n, d))
+        ws_bytes = int(_native.lib().ss_evaluate_workspace(n, d))
 
         def run(time, u, state, spin, ws):
             """Enqueue time evolution and, with a state, the scan (device addresses)."""
