@@ -1416,39 +1416,36 @@ static __device__ __forceinline__ const double* ss_te_sweep(const ss_te_args& a)
 // registers: prefix[row] = the product of the operators of the workgroup's
 // earlier rows, block_total[workgroup] = that of all of them.  u is the row's
 // operator on the first lane of each group of `lanes` (the identity on rows
-// beyond the end); other lanes carry products of theirs that nothing reads.
+// from `end` on); the wave's rows start at `first`.
 // A launch and a read of the operators less than a scan of the stored ones
 // (integrator and states together, without spin): 40 spin-half rows of 10 steps
 // 12.6 -> 8.7 us, 20,000 rows 16.9 -> 14.9, 200,000 rows of 5 33.6 -> 25.2;
 // spin one 21.3 -> 13.2, 28.7 -> 27.8 and 64.3 -> 57.8.
-static __device__ __forceinline__ void ss_scan_block(ss_cd u[SS_D][SS_D], int lanes, bool writes, long long row,
+static __device__ __forceinline__ void ss_scan_block(ss_cd u[SS_D][SS_D], int lanes, long long first, long long end,
                                                      double* prefix, double* block_total)
 {
     __shared__ ss_cd wave_total[4][SS_D][SS_D];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int end = 64 / lanes * lanes;
-#pragma unroll 1
-    for (int s = lanes; s < end; s <<= 1) {
-        ss_cd p[SS_D][SS_D];
+    const int groups = 64 / lanes;
+    if (lanes > 1) {  // row r of the wave to lane r
+        const int from = lane < groups ? lane * lanes : 0;
 #pragma unroll
         for (int r = 0; r < SS_D; ++r)
 #pragma unroll
-            for (int c = 0; c < SS_D; ++c) p[r][c] = ss_c(__shfl_up(u[r][c].x, s, 64), __shfl_up(u[r][c].y, s, 64));
-        if (lane >= s) ss_right_multiply<SS_D>(u, p);
+            for (int c = 0; c < SS_D; ++c)
+                u[r][c] = ss_c(__shfl(u[r][c].x, from, 64), __shfl(u[r][c].y, from, 64));
     }
-    if (lane == end - lanes) ss_copy<SS_D>(u, wave_total[wave]);
+    ss_wave_scan<SS_D>(u, lane, groups);
+    if (lane == groups - 1) ss_copy<SS_D>(u, wave_total[wave]);
     ss_cd ex[SS_D][SS_D], pre[SS_D][SS_D];
-#pragma unroll
-    for (int r = 0; r < SS_D; ++r)
-#pragma unroll
-        for (int c = 0; c < SS_D; ++c)
-            ex[r][c] = ss_c(__shfl_up(u[r][c].x, lanes, 64), __shfl_up(u[r][c].y, lanes, 64));
-    if (lane < lanes) ss_set_identity<SS_D>(ex);
+    ss_dpp_mat<SS_D, SS_DPP_WAVE_SHR1>(u, ex);
+    if (lane == 0) ss_set_identity<SS_D>(ex);
     __syncthreads();
     ss_set_identity<SS_D>(pre);
 #pragma unroll 1
     for (int w = 0; w < wave; ++w) ss_left_multiply<SS_D>(wave_total[w], pre);
     ss_right_multiply<SS_D>(ex, pre);
+    const long long row = first + lane;
     double2* out = reinterpret_cast<double2*>(prefix) + row * (SS_D * SS_D);
     if (threadIdx.x == 192) {
         ss_left_multiply<SS_D>(wave_total[3], pre);
@@ -1458,7 +1455,7 @@ static __device__ __forceinline__ void ss_scan_block(ss_cd u[SS_D][SS_D], int la
 #pragma unroll
             for (int c = 0; c < SS_D; ++c) total[r * SS_D + c] = make_double2(pre[r][c].x, pre[r][c].y);
     }
-    if (writes)
+    if (lane < groups && row < end)
 #pragma unroll
         for (int r = 0; r < SS_D; ++r)
 #pragma unroll
@@ -1473,27 +1470,38 @@ template <bool SCAN>
 static __device__ __forceinline__ void ss_te_item(const ss_te_args& a, const double* sweep, long long item, int p,
                                                   long long first, const ss_ctx* ctx)
 {
-    const int lane = threadIdx.x & 63;
     const int lanes = a.phase_lanes[p];
     const int groups = 64 / lanes;
-    const int gi = lane / lanes;
-    const int rank = lane - gi * lanes;
+    const long long row0 = a.phase_row[p] + (item - first) * groups;
     const long long end = p + 1 < a.n_phases ? a.phase_row[p + 1] : a.n_coarse;
-    const long long row = a.phase_row[p] + (item - first) * groups + gi;
-    const bool active = gi < groups && row < end;
     const int base = a.n_fine / lanes;
     const int rem = a.n_fine - base * lanes;
-    const int j0 = rank * base + (rank < rem ? rank : rem);
-    const int count = active ? base + (rank < rem ? 1 : 0) : 0;
-    const double tc = ss_coarse_time(a.t0, a.dt_out, row);
-    const double rot = active ? ss_rotating_wave(tc, a.dt_out, sweep, ctx) : 0.0;
+    int lane = threadIdx.x & 63;
     ss_cd u[SS_D][SS_D];
-    ss_integrate(u, j0, count, tc, rot, a.dt, a.off_a, a.off_b, sweep, ctx);
+    double rot = 0.0;
+    {
+        const int gi = lane / lanes;
+        const int rank = lane - gi * lanes;
+        const bool active = gi < groups && row0 + gi < end;
+        const int j0 = rank * base + (rank < rem ? rank : rem);
+        const int count = active ? base + (rank < rem ? 1 : 0) : 0;
+        const double tc = ss_coarse_time(a.t0, a.dt_out, row0 + gi);
+        if (active) rot = ss_rotating_wave(tc, a.dt_out, sweep, ctx);
+        ss_integrate(u, j0, count, tc, rot, a.dt, a.off_a, a.off_b, sweep, ctx);
+    }
+    // (the row is worked out again after the steps: kept, it would take
+    // registers from the callback's loop)
+    __asm__("" : "+v"(lane));
+    const int gi = lane / lanes;
+    const int rank = lane - gi * lanes;
+    const long long row = row0 + gi;
+    const bool active = gi < groups && row < end;
     ss_group_reduce(u, rank, lanes);
-    if (active && rank == 0) ss_store(u, rot, a.dt_out, tc, row, a.time_out, a.u_out);
+    if (active && rank == 0)
+        ss_store(u, rot, a.dt_out, ss_coarse_time(a.t0, a.dt_out, row), row, a.time_out, a.u_out);
     if (SCAN && a.prefix) {
         if (!active) ss_set_identity<SS_D>(u);
-        ss_scan_block(u, lanes, active && rank == 0, row, a.prefix, a.block_total);
+        ss_scan_block(u, lanes, row0, end, a.prefix, a.block_total);
     }
 }
 
@@ -1503,7 +1511,7 @@ extern "C" __global__ void SS_KERNEL_ATTR ss_time_evolution_kernel(ss_te_args a)
 {
     ss_trig_load();
     ss_exp_load();
-    const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const long long wave = (long long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (wave >= a.items && !a.prefix) return;  // whole waves only
     ss_ctx ctx;
     ctx.tables = reinterpret_cast<const ss_table*>(a.tables);

@@ -158,42 +158,13 @@ constexpr int kSingleScanBlock = 256;
 // reads 64 (spin one: 144) KiB of totals and the gain is still 18 (11) %.
 constexpr int kFusedScanBlocks = 1024;
 
-template <int D>
-__device__ __forceinline__ void shfl_down_mat(const ss_cd m[D][D], ss_cd out[D][D], int s)
-{
-#pragma unroll
-    for (int r = 0; r < D; ++r)
-#pragma unroll
-        for (int c = 0; c < D; ++c) {
-            out[r][c].x = __shfl_down(m[r][c].x, s, 64);
-            out[r][c].y = __shfl_down(m[r][c].y, s, 64);
-        }
-}
-
-template <int D>
-__device__ __forceinline__ void shfl_up_mat(const ss_cd m[D][D], ss_cd out[D][D], int s)
-{
-#pragma unroll
-    for (int r = 0; r < D; ++r)
-#pragma unroll
-        for (int c = 0; c < D; ++c) {
-            out[r][c].x = __shfl_up(m[r][c].x, s, 64);
-            out[r][c].y = __shfl_up(m[r][c].y, s, 64);
-        }
-}
-
 // Inclusive scan over the 64 lanes of a wave of x_l (later lanes on the
 // left): q_l = x_l x_{l-1} ... x_0.  Then ex = q_{l-1} (identity on lane 0).
 template <int D>
 __device__ __forceinline__ void wave_scan(ss_cd q[D][D], ss_cd ex[D][D], int lane)
 {
-#pragma unroll 1
-    for (int s = 1; s < 64; s <<= 1) {
-        ss_cd p[D][D];
-        shfl_up_mat<D>(q, p, s);
-        if (lane >= s) ss_right_multiply<D>(q, p);
-    }
-    shfl_up_mat<D>(q, ex, 1);
+    ss_wave_scan<D>(q, lane, 64);
+    ss_dpp_mat<D, SS_DPP_WAVE_SHR1>(q, ex);
     if (lane == 0) ss_set_identity<D>(ex);
 }
 
@@ -302,8 +273,7 @@ __global__ void __launch_bounds__(kSingleScanBlock) single_scan_apply(const doub
 }
 
 // Carry-in state of this workgroup, v_b = (T_{b-1} ... T_0) psi0, from the
-// totals before it: consecutive ones per thread, an ordered shuffle tree per
-// wave, the four wave products through LDS.  Each workgroup forms its own, so
+// totals before it: consecutive ones per thread, a scan per wave, the four wave products through LDS.  Each workgroup forms its own, so
 // no pass of one workgroup stands between the totals and the states.
 template <int D>
 __device__ __forceinline__ void block_carry(const double* block_total, ss_cd p0, ss_cd p1, ss_cd p2, ss_cd c[D])
@@ -319,20 +289,16 @@ __device__ __forceinline__ void block_carry(const double* block_total, ss_cd p0,
         load_mat<D>(block_total, b, tot);
         ss_left_multiply<D>(tot, m);
     }
-    // product over the wave's lanes, later totals on the left (lanes from the
-    // workgroup's number on hold the identity)
-#pragma unroll 1
-    for (int s = 1; s < 64 && s < (int)blockIdx.x; s <<= 1) {
-        ss_cd o[D][D];
-        shfl_down_mat<D>(m, o, s);
-        if ((lane & (2 * s - 1)) == 0) ss_left_multiply<D>(o, m);
-    }
-    if (lane == 0) ss_copy<D>(m, wave_prod[wave]);
+    // product over the wave's lanes that have totals, later ones on the left
+    const int used = per ? ((int)blockIdx.x + per - 1) / per : 0;
+    const int count = used - 64 * wave < 64 ? used - 64 * wave : 64;
+    ss_wave_scan<D>(m, lane, count);
+    if (lane == (count > 1 ? count - 1 : 0)) ss_copy<D>(m, wave_prod[wave]);
     __syncthreads();
     if (t == 0) {
         ss_cd pr[D][D];
         ss_copy<D>(wave_prod[0], pr);
-        for (int w = 1; w < kSingleScanBlock / 64 && 64 * w * per < (int)blockIdx.x; ++w)
+        for (int w = 1; 64 * w < used; ++w)
             ss_left_multiply<D>(wave_prod[w], pr);
         const ss_cd psi[3] = {p0, p1, p2};
         ss_cd v[D];
@@ -402,11 +368,11 @@ __global__ void __launch_bounds__(kSingleScanBlock) evaluate_states(const double
 // leading into r, or, where r starts a simulation, v -> init (an affine map
 // v -> m v + c with m = 0).  The rows are cut into chunks of whole 256-row
 // tiles, one workgroup per chunk.  Pass 1 composes each chunk's maps (a wave
-// shuffle reduction per tile, tiles in order) and stores the chunk's map.
+// scan per tile, tiles in order) and stores the chunk's map.
 // Pass 2 finds each chunk's incoming state from the maps of the chunks before
 // it, back to the nearest one in which a simulation starts (up to 256 chunks
-// per look, multiplied in order by a shuffle tree), then walks its own tiles:
-// a wave shuffle scan plus the four wave totals through LDS gives each row its
+// per look, multiplied in order by a wave scan), then walks its own tiles:
+// a wave scan plus the four wave totals through LDS gives each row its
 // state from the tile's incoming one, written with its Bloch vector.  No
 // workgroup waits on another: pass 2 starts after pass 1 has finished.
 
@@ -480,7 +446,7 @@ __device__ __forceinline__ void load_vec_c(const double* p, ss_cd v[D])
 // U[total - r]^+ backward (costate[i] = U[i+1]^+ costate[i+1]).
 // Q (spin half, special unitary operators): every map matrix has the form
 // [[p, -conj q], [q, conj p]] (operators, their products, identity and zero),
-// kept expanded in registers but computed and shuffled as its first column.
+// kept expanded in registers but computed and moved as its first column.
 template <int D>
 __device__ __forceinline__ void su2_expand(ss_cd m[D][D], ss_cd p, ss_cd q)
 {
@@ -620,24 +586,28 @@ __device__ __forceinline__ void aff_before(ss_cd m[D][D], ss_cd c[D], const ss_c
     }
 }
 
-template <int D, bool AFF, bool UP, bool Q = false>
-__device__ __forceinline__ void shfl_aff(const ss_cd m[D][D], const ss_cd c[D], ss_cd om[D][D], ss_cd oc[D], int s)
+template <int D, bool AFF, int CTRL, bool Q>
+__device__ __forceinline__ void dpp_aff(const ss_cd m[D][D], const ss_cd c[D], ss_cd om[D][D], ss_cd oc[D])
 {
 #pragma unroll
     for (int r = 0; r < D; ++r) {
 #pragma unroll
-        for (int k = 0; k < ((Q && D == 2) ? 1 : D); ++k) {
-            om[r][k].x = UP ? __shfl_up(m[r][k].x, s, 64) : __shfl_down(m[r][k].x, s, 64);
-            om[r][k].y = UP ? __shfl_up(m[r][k].y, s, 64) : __shfl_down(m[r][k].y, s, 64);
-        }
-        if (AFF) {
-            oc[r].x = UP ? __shfl_up(c[r].x, s, 64) : __shfl_down(c[r].x, s, 64);
-            oc[r].y = UP ? __shfl_up(c[r].y, s, 64) : __shfl_down(c[r].y, s, 64);
-        } else {
-            oc[r] = ss_c(0.0, 0.0);
-        }
+        for (int k = 0; k < ((Q && D == 2) ? 1 : D); ++k)
+            om[r][k] = ss_c(ss_dpp<CTRL>(m[r][k].x), ss_dpp<CTRL>(m[r][k].y));
+        oc[r] = AFF ? ss_c(ss_dpp<CTRL>(c[r].x), ss_dpp<CTRL>(c[r].y)) : ss_c(0.0, 0.0);
     }
     if constexpr (Q && D == 2) su2_expand<D>(om, om[0][0], om[1][0]);
+}
+
+// Inclusive scan over the 64 lanes of a wave: q_l <- q_l o q_{l-1} o ... o q_0.
+template <int D, bool AFF, bool Q>
+__device__ __forceinline__ void wave_scan_aff(ss_cd qm[D][D], ss_cd qc[D], int lane)
+{
+    ss_scan_steps(lane, 64, [&](auto ctrl, bool applies) {
+        ss_cd pm[D][D], pc[D];
+        dpp_aff<D, AFF, decltype(ctrl)::value, Q>(qm, qc, pm, pc);
+        if (applies) aff_before<D, AFF, Q>(qm, qc, pm, pc);
+    });
 }
 
 struct ScanShared {
@@ -781,14 +751,8 @@ __device__ void scan_tile_reduce(const ScanArgs& a, long long r0, long long r1, 
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     ss_cd xm[D][D], xc[D];
     scan_thread_map<D, REV, R, AFF, Q>(a, r0, r1, start_sim, xm, xc);
-    // x_l <- x_{l+s} o x_l: lane 0 ends with the wave's map (later rows on the left)
-#pragma unroll 1
-    for (int s = 1; s < 64; s <<= 1) {
-        ss_cd om[D][D], oc[D];
-        shfl_aff<D, AFF, false, Q>(xm, xc, om, oc, s);
-        if ((lane & (2 * s - 1)) == 0) aff_after<D, AFF, Q>(om, oc, xm, xc);
-    }
-    if (lane == 0) {
+    wave_scan_aff<D, AFF, Q>(xm, xc, lane);
+    if (lane == 63) {
         ss_copy<D>(xm, s_tm[w]);
 #pragma unroll
         for (int r = 0; r < D; ++r) s_tc[w][r] = xc[r];
@@ -882,19 +846,13 @@ __device__ void scan_incoming(const ScanArgs& a, long long j, ss_cd vin[D], Scan
         const int pm = sh.pmin;
         if (t < pm) load_mat_at<D>(a.agg + idx * kStride, m);
         // ordered product m_0 m_1 ... m_{pm-1}, chunk k on the left
-#pragma unroll 1
-        for (int s = 1; s < 64; s <<= 1) {
+        const int count = pm - 64 * w < 64 ? pm - 64 * w : 64;
+        ss_scan_steps(lane, count, [&](auto ctrl, bool applies) {
             ss_cd o[D][D];
-#pragma unroll
-            for (int r = 0; r < D; ++r)
-#pragma unroll
-                for (int c = 0; c < D; ++c) {
-                    o[r][c].x = __shfl_down(m[r][c].x, s, 64);
-                    o[r][c].y = __shfl_down(m[r][c].y, s, 64);
-                }
-            if ((lane & (2 * s - 1)) == 0 && lane + s < 64) ss_right_multiply<D>(m, o);
-        }
-        if (lane == 0) ss_copy<D>(m, s_m[w]);
+            ss_dpp_mat<D, decltype(ctrl)::value>(m, o);
+            if (applies) ss_left_multiply<D>(o, m);
+        });
+        if (lane == (count > 1 ? count - 1 : 0)) ss_copy<D>(m, s_m[w]);
         if (pm < kScanThreads && t == pm) {
             if (idx >= 0) {
                 load_vec_c<D>(a.agg + idx * kStride + 2 * D * D, s_v);
@@ -905,7 +863,7 @@ __device__ void scan_incoming(const ScanArgs& a, long long j, ss_cd vin[D], Scan
         }
         __syncthreads();
 #pragma unroll 1
-        for (int ww = 0; ww < 4; ++ww) ss_right_multiply<D>(acc, s_m[ww]);
+        for (int ww = 0; 64 * ww < pm; ++ww) ss_right_multiply<D>(acc, s_m[ww]);
         const bool done = pm < kScanThreads;
         if (done) ss_matvec<D>(acc, s_v, vin);
         __syncthreads();
@@ -922,13 +880,7 @@ __device__ void scan_tile_apply(const ScanArgs& a, long long r0, long long r1, c
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     ss_cd qm[D][D], qc[D];
     scan_thread_map<D, REV, R, AFF, Q>(a, r0, r1, start_sim, qm, qc);
-    // inclusive scan over the wave: q_l <- q_l o q_{l-s}
-#pragma unroll 1
-    for (int s = 1; s < 64; s <<= 1) {
-        ss_cd pm[D][D], pc[D];
-        shfl_aff<D, AFF, true, Q>(qm, qc, pm, pc, s);
-        if (lane >= s) aff_before<D, AFF, Q>(qm, qc, pm, pc);
-    }
+    wave_scan_aff<D, AFF, Q>(qm, qc, lane);
     if (lane == 63) {
         ss_copy<D>(qm, s_tm[w]);
 #pragma unroll
@@ -937,7 +889,7 @@ __device__ void scan_tile_apply(const ScanArgs& a, long long r0, long long r1, c
     if (R > 1) {
         // exclusive: the rows of earlier lanes of the wave
         ss_cd em[D][D], ec[D];
-        shfl_aff<D, AFF, true, Q>(qm, qc, em, ec, 1);
+        dpp_aff<D, AFF, SS_DPP_WAVE_SHR1, Q>(qm, qc, em, ec);
         if (lane == 0) {
             ss_set_identity<D>(em);
             set_zero_vec<D>(ec);
@@ -1725,7 +1677,7 @@ int launch_scan(const char* who, ScanArgs a, int dim, bool reverse, int64_t chun
     // kScanRows rows per thread when each chunk is one tile (latency-bound)
     const bool wide = l.chunk_rows > kScanTileRows;
     if (dim == 2 && !reverse && a.u_layout != SS_U_FULL) {
-        // special unitary operators: maps composed and shuffled as first
+        // special unitary operators: maps composed and moved as first
         // columns.  Pass 1 over wide chunks reads 64 bytes of rows per lane
         // (two first-column rows, or one full row whose first column it
         // reads): the lanes' loads then share cache lines, where four rows a
