@@ -378,6 +378,11 @@ __global__ void __launch_bounds__(kSingleScanBlock) evaluate_states(const double
 
 constexpr int kScanThreads = 256;
 
+// Rows per thread of the state scan; a tile is 256 threads.
+constexpr int kScanRows = 4;
+
+constexpr long long kScanTileRows = 256LL * kScanRows;
+
 struct ScanArgs {
     const double* u;            // (total, D, D), or (total, 2) first columns with u_layout 1
     double* out;                // (total, D) states, or costates
@@ -969,6 +974,24 @@ __global__ void __launch_bounds__(kScanThreads) batch_scan_apply(ScanArgs a)
     }
 }
 
+// Both passes, with R1 and R2 rows per thread.
+template <int D, bool REV, bool Q, int R1, int R2>
+void launch_scan_passes(const ScanArgs& a, dim3 g, dim3 b, hipStream_t s)
+{
+    hipLaunchKernelGGL((batch_scan_reduce<D, REV, R1, Q>), g, b, 0, s, a);
+    hipLaunchKernelGGL((batch_scan_apply<D, REV, R2, Q>), g, b, 0, s, a);
+}
+
+// The rows per thread of one-tile chunks, or (0) those of larger ones.
+template <int D, bool REV, bool Q>
+void launch_scan_passes(const ScanArgs& a, int rows, dim3 g, dim3 b, hipStream_t s)
+{
+    if (rows == 1) launch_scan_passes<D, REV, Q, 1, 1>(a, g, b, s);
+    else if (rows == 2) launch_scan_passes<D, REV, Q, 2, 2>(a, g, b, s);
+    else if (rows) launch_scan_passes<D, REV, Q, kScanRows, kScanRows>(a, g, b, s);
+    else launch_scan_passes<D, REV, Q, kScanRows, 1>(a, g, b, s);
+}
+
 // psi(T) of each simulation: U[last] state[last] (psi0 when it has no rows).
 template <int D>
 __global__ void __launch_bounds__(256) final_state_kernel(const double* psi0, const double* u, const double* state,
@@ -1101,20 +1124,26 @@ struct ScanLayout {
     size_t bytes;
 };
 
-// Rows per thread of the state scan; a tile is 256 threads.
-constexpr int kScanRows = 4;
-
-constexpr long long kScanTileRows = 256LL * kScanRows;
-
 // Chunks of whole tiles: `chunk_rows` rows each (a positive multiple of the
 // 1024-row tile), or by default at most about 2048 chunks (8 workgroups per
-// CU).  The workspace holds one record (map and constant flag) per chunk.
+// CU).  Small scans are bound by the serial work of a tile, so while one
+// workgroup a CU (spin half: two, whose products leave the vector units free)
+// covers the rows, a thread takes one row in chunks of 256, else two in chunks
+// of 512.  Scans of 1000, 65,536, 100,000 and 200,000 rows in simulations of
+// 3000: spin half 18.2 -> 12.2, 23.4 -> 15.7, 24.2 -> 16.6, 26.3 -> 22.6 us, spin
+// one 24.5 -> 17.4, 30.9 -> 22.6, 31.4 -> 25.9 and (four rows a thread still; two
+// gain 6 % forward and lose as much backward) 37.5.
+// The workspace holds one record (map and constant flag) per chunk.
 ScanLayout scan_layout(int64_t n, int dim, int64_t chunk_rows = 0)
 {
     ScanLayout l{};
     l.tiles = (n + kScanTileRows - 1) / kScanTileRows;
     if (chunk_rows > 0) {
         l.chunk_rows = chunk_rows;
+    } else if (n <= (dim == 2 ? 131072 : 65536)) {
+        l.chunk_rows = kScanThreads;
+    } else if (n <= (dim == 2 ? 262144 : 131072)) {
+        l.chunk_rows = 2 * kScanThreads;
     } else {
         const long long per = std::max(1LL, (l.tiles + 2047) / 2048);
         l.chunk_rows = kScanTileRows * per;
@@ -1673,9 +1702,9 @@ int launch_scan(const char* who, ScanArgs a, int dim, bool reverse, int64_t chun
     a.n_chunks = l.chunks;
     const dim3 g(unsigned(l.chunks)), b(kScanThreads);
     // pass 2 with one row per thread once chunks span several tiles (large,
-    // bandwidth-bound scans: row-contiguous lanes store coalesced); with
-    // kScanRows rows per thread when each chunk is one tile (latency-bound)
-    const bool wide = l.chunk_rows > kScanTileRows;
+    // bandwidth-bound scans: row-contiguous lanes store coalesced); with a
+    // tile's rows per thread when each chunk is one tile (latency-bound)
+    const int rows = l.chunk_rows > kScanTileRows ? 0 : int(l.chunk_rows / kScanThreads);
     if (dim == 2 && !reverse && a.u_layout != SS_U_FULL) {
         // special unitary operators: maps composed and moved as first
         // columns.  Pass 1 over wide chunks reads 64 bytes of rows per lane
@@ -1685,30 +1714,20 @@ int launch_scan(const char* who, ScanArgs a, int dim, bool reverse, int64_t chun
         // requests -- 1.02 -> 0.83 ms (first columns) and 1.52 -> 1.28 ms
         // (full rows) for 1.06e8 rows; spin one keeps four rows a lane (one
         // a lane: 2.2 -> 2.7 ms for its scans of 2e7 rows)
-        if (!wide)
-            hipLaunchKernelGGL((batch_scan_reduce<2, false, kScanRows, true>), g, b, 0, s, a);
+        if (rows)
+            launch_scan_passes<2, false, true>(a, rows, g, b, s);
         else if (a.u_layout == SS_U_SU2_COLUMN)
-            hipLaunchKernelGGL((batch_scan_reduce<2, false, 2, true>), g, b, 0, s, a);
+            launch_scan_passes<2, false, true, 2, 1>(a, g, b, s);
         else
-            hipLaunchKernelGGL((batch_scan_reduce<2, false, 1, true>), g, b, 0, s, a);
-        if (wide) hipLaunchKernelGGL((batch_scan_apply<2, false, 1, true>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((batch_scan_apply<2, false, kScanRows, true>), g, b, 0, s, a);
+            launch_scan_passes<2, false, true, 1, 1>(a, g, b, s);
     } else if (dim == 2 && !reverse) {
-        hipLaunchKernelGGL((batch_scan_reduce<2, false, kScanRows>), g, b, 0, s, a);
-        if (wide) hipLaunchKernelGGL((batch_scan_apply<2, false, 1>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((batch_scan_apply<2, false, kScanRows>), g, b, 0, s, a);
+        launch_scan_passes<2, false, false>(a, rows, g, b, s);
     } else if (dim == 3 && !reverse) {
-        hipLaunchKernelGGL((batch_scan_reduce<3, false, kScanRows>), g, b, 0, s, a);
-        if (wide) hipLaunchKernelGGL((batch_scan_apply<3, false, 1>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((batch_scan_apply<3, false, kScanRows>), g, b, 0, s, a);
+        launch_scan_passes<3, false, false>(a, rows, g, b, s);
     } else if (dim == 2) {
-        hipLaunchKernelGGL((batch_scan_reduce<2, true, kScanRows>), g, b, 0, s, a);
-        if (wide) hipLaunchKernelGGL((batch_scan_apply<2, true, 1>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((batch_scan_apply<2, true, kScanRows>), g, b, 0, s, a);
+        launch_scan_passes<2, true, false>(a, rows, g, b, s);
     } else {
-        hipLaunchKernelGGL((batch_scan_reduce<3, true, kScanRows>), g, b, 0, s, a);
-        if (wide) hipLaunchKernelGGL((batch_scan_apply<3, true, 1>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((batch_scan_apply<3, true, kScanRows>), g, b, 0, s, a);
+        launch_scan_passes<3, true, false>(a, rows, g, b, s);
     }
     SS_HIP(hipGetLastError());
     return 0;
