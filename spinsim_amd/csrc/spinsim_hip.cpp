@@ -1041,16 +1041,33 @@ __global__ void __launch_bounds__(256) adjoint_reduce_windows(const double* part
     for (int c = 0; c < n_controls; ++c) {
         const long long k = j - ctl[c].grad_offset;
         if (k < 0 || k >= tables[ctl[c].table].size) continue;
-        // first row whose window reaches knot k: base + W > k
-        long long lo = r0, hi = r1;
-        while (lo < hi) {
-            const long long mid = (lo + hi) >> 1;
-            if (window_base[mid * n_controls + c] + SS_ADJ_WINDOW > k) hi = mid; else lo = mid + 1;
+        // rows [lo, top): from the first whose window reaches knot k (base + W >
+        // k) to the first whose window starts after it, both searches at once
+        long long lo = r0, hi = r1, top = r0, end = r1;
+        while (lo < hi || top < end) {
+            const long long mid = (lo + hi) >> 1, mid2 = (top + end) >> 1;
+            const long long b = lo < hi ? window_base[mid * n_controls + c] : 0;
+            const long long b2 = top < end ? window_base[mid2 * n_controls + c] : 0;
+            if (lo < hi) {
+                if (b + SS_ADJ_WINDOW > k) hi = mid; else lo = mid + 1;
+            }
+            if (top < end) {
+                if (b2 > k) end = mid2; else top = mid2 + 1;
+            }
         }
-        for (long long r = lo; r < r1; ++r) {
-            const long long b = window_base[r * n_controls + c];
-            if (b > k) break;
-            sum += partial[(r * n_controls + c) * SS_ADJ_WINDOW + (k - b)];
+        // added in row order, read eight rows at a time: the loop is bound by
+        // the latency of its two loads, base and entry (24 simulations of 333
+        // rows and 97 knots of three controls: 32 -> 21 us)
+        for (long long r = lo; r < top; r += 8) {
+            double v[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const long long rq = r + q < top ? r + q : lo;
+                v[q] = partial[(rq * n_controls + c) * SS_ADJ_WINDOW + (k - window_base[rq * n_controls + c])];
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                if (r + q < top) sum += v[q];
         }
     }
     grad[i] = sum;
