@@ -179,15 +179,18 @@ int ss_time_evolution(const ss_module *m, const double *sweep, double t0, double
 /* evaluate() of one simulation in one call (spinsim/__init__.py:993-1085):
  * ss_time_evolution with 1 to 32 sweep parameters given in HOST memory (they
  * travel in the kernel arguments, so nothing is copied and the array may be
- * reused at once), then, unless state is NULL, ss_state_scan of its operators
+ * reused at once; n_sweep 0: sweep is a device array, as there), then, unless state is NULL, ss_state_scan of its operators
  * (psi0 in host memory; spin NULL or (n, 3); a workspace of that call's size).
  * With a workspace of ss_evaluate_workspace bytes the integrator leaves the
- * scan's products itself where its launch has at most 1024 workgroups, and one
- * pass writes the states. */
+ * scan's products itself where its launch has at most 16,384 workgroups, and one
+ * pass writes the states (beyond 1024, after one for the carries).  reader:
+ * NULL, or a stream that then waits for the operators and times (to copy them
+ * while the states are formed). */
 int ss_evaluate(const ss_module *m, const double *sweep, int n_sweep, double t0, double dt,
                 double dt_out, int64_t n_coarse, double *time_out, double *u_out,
                 const ss_table *tables, int lanes_per_step, const double *psi0, double *state,
-                double *spin, void *workspace, size_t workspace_bytes, ss_stream stream);
+                double *spin, void *workspace, size_t workspace_bytes, ss_stream stream,
+                ss_stream reader);
 size_t ss_evaluate_workspace(int64_t n, int dim);
 /* Lanes per coarse step of the default launch for n_rows rows of n_fine steps
  * on `cus` compute units that hold `resident` workgroups each (host only; 1..64,

@@ -40,7 +40,7 @@ SIGNATURES = {
     "ss_time_evolution": (c_int, [c_vp, c_vp, c_dbl, c_dbl, c_dbl, c_i64, c_vp, c_vp, c_vp,
                                   c_int, c_vp]),
     "ss_evaluate": (c_int, [c_vp, c_vp, c_int, c_dbl, c_dbl, c_dbl, c_i64, c_vp, c_vp, c_vp, c_int,
-                            c_vp, c_vp, c_vp, c_vp, ctypes.c_size_t, c_vp]),
+                            c_vp, c_vp, c_vp, c_vp, ctypes.c_size_t, c_vp, c_vp]),
     "ss_batch_time_evolution": (c_int, [c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_vp,
                                         c_i64, c_vp, c_vp, c_vp, c_vp, c_int, c_int, c_int,
                                         c_int, c_vp]),

@@ -157,6 +157,14 @@ constexpr int kSingleScanBlock = 256;
 // workgroups: 17.9 -> 14.8 us; spin one 33.3 -> 29.0).  At the limit each
 // reads 64 (spin one: 144) KiB of totals and the gain is still 18 (11) %.
 constexpr int kFusedScanBlocks = 1024;
+// Workgroups up to which ss_evaluate's integrator leaves the products (beyond
+// kFusedScanBlocks one workgroup scans their totals, a few microseconds for each
+// thousand; with several lanes a row its workgroups hold fewer rows, and the
+// scan of the stored operators is the shorter one: 190 against 195 us for 1191
+// workgroups of 84 rows, integrator included).  700,000 spin-half rows 72 -> 62
+// us against the scan of stored operators, 4e6 rows 358 -> 353; spin one 142 ->
+// 126 and 759 -> 744.
+constexpr long long kEvaluateBlocks = 16384;
 
 // Inclusive scan over the 64 lanes of a wave of x_l (later lanes on the
 // left): q_l = x_l x_{l-1} ... x_0.  Then ex = q_{l-1} (identity on lane 0).
@@ -345,20 +353,47 @@ __global__ void __launch_bounds__(kSingleScanBlock) single_scan_apply_carry(cons
 // The states of a time evolution that left its products (ss_scan_block of the
 // integrator): workgroup b holds rows [rows * b, rows * b + rows), and
 // state[k] = prefix[k] v_b.
-template <int D>
+// v_b comes from the totals, or from single_scan_blocks.
+template <int D, bool CARRY>
 __global__ void __launch_bounds__(kSingleScanBlock) evaluate_states(const double* prefix, long long n, int rows,
-                                                         const double* block_total, ss_cd p0, ss_cd p1,
-                                                         ss_cd p2, double* state, double* spin)
+                                                         const double* block_total, const double* carry,
+                                                         ss_cd p0, ss_cd p1, ss_cd p2, double* state,
+                                                         double* spin)
 {
     const long long k = (long long)blockIdx.x * rows + threadIdx.x;
     const bool active = (int)threadIdx.x < rows && k < n;
     ss_cd pre[D][D], c[D], v[D];
     if (active) load_mat<D>(prefix, k, pre);
-    block_carry<D>(block_total, p0, p1, p2, c);
+    if (CARRY) load_vec<D>(carry, blockIdx.x, c);
+    else block_carry<D>(block_total, p0, p1, p2, c);
     if (!active) return;
     ss_matvec<D>(pre, c, v);
     store_vec<D>(state, k, v);
     if (spin) ss_store_spin<D>(v, spin, k);
+}
+
+// Where a time evolution may leave its operators' products (workspace of
+// evaluate_layout), and what it left: the launch's workgroups, 0 for no products,
+// and the rows of each.
+struct EvaluateScan {
+    double *prefix, *block_total;
+    long long blocks;
+    int rows;
+};
+
+template <int D>
+void launch_evaluate_states(const EvaluateScan& e, double* carry, long long n, ss_cd p0, ss_cd p1, ss_cd p2,
+                            double* state, double* spin, hipStream_t s)
+{
+    const dim3 grid(unsigned(e.blocks)), block(kSingleScanBlock);
+    if (e.blocks <= kFusedScanBlocks) {
+        hipLaunchKernelGGL((evaluate_states<D, false>), grid, block, 0, s, e.prefix, n, e.rows, e.block_total, carry,
+                           p0, p1, p2, state, spin);
+    } else {
+        hipLaunchKernelGGL(single_scan_blocks<D>, dim3(1), block, 0, s, e.block_total, e.blocks, p0, p1, p2, carry);
+        hipLaunchKernelGGL((evaluate_states<D, true>), grid, block, 0, s, e.prefix, n, e.rows, e.block_total, carry,
+                           p0, p1, p2, state, spin);
+    }
 }
 
 // ---- state scan: get_state (:1087-1111) batches and costates, two passes -----
@@ -1129,11 +1164,20 @@ SingleScanLayout single_scan_layout(int64_t n, int dim)
     return l;
 }
 
-// Workspace of ss_evaluate's scan: a product per row, a total per workgroup.
-size_t evaluate_total_off(int64_t n, int dim) { return align256(size_t(n) * dim * dim * 16); }
-size_t evaluate_bytes(int64_t n, int dim)
+// Workspace of ss_evaluate's scan: a product per row, a total and a carry per
+// workgroup (of at least four rows).
+struct EvaluateLayout {
+    size_t total_off, carry_off, bytes;
+};
+
+EvaluateLayout evaluate_layout(int64_t n, int dim)
 {
-    return evaluate_total_off(n, dim) + align256(size_t(kFusedScanBlocks) * dim * dim * 16);
+    const size_t vec = size_t(dim) * 16, groups = size_t(std::min<int64_t>((n + 3) / 4, kEvaluateBlocks));
+    EvaluateLayout l;
+    l.total_off = align256(size_t(n) * dim * vec);
+    l.carry_off = l.total_off + align256(groups * dim * vec);
+    l.bytes = l.carry_off + align256(groups * vec);
+    return l;
 }
 
 struct ScanLayout {
@@ -1522,15 +1566,6 @@ int ss_time_evolution_plan(int64_t n_coarse, int n_fine, int64_t waves, int* n_p
     return 0;
 }
 
-// Where a time evolution may leave its operators' products (workspace of
-// evaluate_bytes), and what it left: the launch's workgroups, 0 for no products,
-// and the rows of each.
-struct EvaluateScan {
-    double *prefix, *block_total;
-    long long blocks;
-    int rows;
-};
-
 // ss_time_evolution with the sweep parameters in a device array, or (sweep null)
 // n_inline of them in host memory, which go into the kernel arguments.
 static int time_evolution(const char* who, const ss_module* m, const double* sweep, const double* sweep_host,
@@ -1577,7 +1612,7 @@ static int time_evolution(const char* who, const ss_module* m, const double* swe
     }
     const long long blocks = (a.waves + 3) / 4;
     if (blocks > 2147483647LL) return fail("%s: grid too large", who);
-    if (scan && lanes_per_step > 0 && blocks <= kFusedScanBlocks) {
+    if (scan && lanes_per_step > 0 && blocks <= (lanes_per_step == 1 ? kEvaluateBlocks : kFusedScanBlocks)) {
         a.prefix = scan->prefix;
         a.block_total = scan->block_total;
         scan->blocks = blocks;
@@ -1600,40 +1635,49 @@ size_t ss_evaluate_workspace(int64_t n, int dim)
 {
     if (n <= 0 || (dim != 2 && dim != 3)) return 0;
     const size_t scan = ss_state_scan_workspace(n, dim);
-    return n <= kFusedScanBlocks * 256LL ? std::max(scan, evaluate_bytes(n, dim)) : scan;
+    return n <= kEvaluateBlocks * 256 ? std::max(scan, evaluate_layout(n, dim).bytes) : scan;
 }
 
 int ss_evaluate(const ss_module* m, const double* sweep, int n_sweep, double t0, double dt, double dt_out,
                 int64_t n_coarse, double* time_out, double* u_out, const ss_table* tables, int lanes_per_step,
                 const double* psi0, double* state, double* spin, void* workspace, size_t workspace_bytes,
-                ss_stream stream)
+                ss_stream stream, ss_stream reader)
 {
-    if (n_sweep < 1 || n_sweep > SS_SWEEP_INLINE) {
+    if (n_sweep < 0 || n_sweep > SS_SWEEP_INLINE) {
         (void)take_te_events();
-        return fail("ss_evaluate: 1 to %d sweep parameters, got %d", SS_SWEEP_INLINE, n_sweep);
+        return fail("ss_evaluate: 0 to %d sweep parameters in host memory, got %d", SS_SWEEP_INLINE, n_sweep);
     }
-    // up to kFusedScanBlocks workgroups the integrator does the scan's first pass
+    // up to kEvaluateBlocks workgroups the integrator does the scan's first pass
     EvaluateScan scan = {};
-    if (m && psi0 && state && workspace && n_coarse > 0 && n_coarse <= kFusedScanBlocks * 256LL &&
-        workspace_bytes >= evaluate_bytes(n_coarse, m->dim)) {
-        scan.prefix = static_cast<double*>(workspace);
-        scan.block_total = reinterpret_cast<double*>(static_cast<char*>(workspace) + evaluate_total_off(n_coarse, m->dim));
+    double* carry = nullptr;
+    if (m && psi0 && state && workspace && n_coarse > 0 && n_coarse <= kEvaluateBlocks * 256) {
+        const EvaluateLayout l = evaluate_layout(n_coarse, m->dim);
+        if (workspace_bytes >= l.bytes) {
+            char* ws = static_cast<char*>(workspace);
+            scan.prefix = reinterpret_cast<double*>(ws);
+            scan.block_total = reinterpret_cast<double*>(ws + l.total_off);
+            carry = reinterpret_cast<double*>(ws + l.carry_off);
+        }
     }
-    if (int rc = time_evolution("ss_evaluate", m, nullptr, sweep, n_sweep, t0, dt, dt_out, n_coarse, time_out, u_out,
-                                tables, lanes_per_step, scan.prefix ? &scan : nullptr, stream))
+    if (int rc = time_evolution("ss_evaluate", m, n_sweep ? nullptr : sweep, sweep, n_sweep, t0, dt, dt_out, n_coarse,
+                                time_out, u_out, tables, lanes_per_step, scan.prefix ? &scan : nullptr, stream))
         return rc;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (reader && n_coarse > 0) {
+        hipEvent_t ready;
+        SS_HIP(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
+        hipError_t e = hipEventRecord(ready, s);
+        if (e == hipSuccess) e = hipStreamWaitEvent(static_cast<hipStream_t>(reader), ready, 0);
+        (void)hipEventDestroy(ready);
+        if (e != hipSuccess) return fail("ss_evaluate: %s", hipGetErrorString(e));
+    }
     if (!state) return 0;
-    if (!scan.blocks) return ss_state_scan(psi0, u_out, state, spin, n_coarse, m->dim, workspace, workspace_bytes, stream);
+    if (!scan.blocks)
+        return ss_state_scan(psi0, u_out, state, spin, n_coarse, m->dim, workspace, workspace_bytes, stream);
     const ss_cd p0 = ss_c(psi0[0], psi0[1]), p1 = ss_c(psi0[2], psi0[3]);
     const ss_cd p2 = m->dim == 3 ? ss_c(psi0[4], psi0[5]) : ss_c(0, 0);
-    const dim3 grid(unsigned(scan.blocks)), block(kSingleScanBlock);
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (m->dim == 2)
-        hipLaunchKernelGGL(evaluate_states<2>, grid, block, 0, s, scan.prefix, (long long)n_coarse, scan.rows,
-                           scan.block_total, p0, p1, p2, state, spin);
-    else
-        hipLaunchKernelGGL(evaluate_states<3>, grid, block, 0, s, scan.prefix, (long long)n_coarse, scan.rows,
-                           scan.block_total, p0, p1, p2, state, spin);
+    if (m->dim == 2) launch_evaluate_states<2>(scan, carry, n_coarse, p0, p1, p2, state, spin, s);
+    else launch_evaluate_states<3>(scan, carry, n_coarse, p0, p1, p2, state, spin, s);
     SS_HIP(hipGetLastError());
     return 0;
 }

@@ -416,11 +416,14 @@ class Simulator:
         self._launch_time_evolution(sweep, t0, dt, dt_out, int(time_out.shape[0]), dev,
                                     time_out.data_ptr(), u_out.data_ptr(), lanes, stream)
 
+    def _tuned_lanes(self, sweep, t0, dt, dt_out, n):
+        from .autotune import tune_lanes
+        n_fine = math.floor(dt_out / dt + 0.5)
+        return tune_lanes(self, n, n_fine, dt, dt_out, sweep, t0)[0] if n else 0
+
     def _launch_time_evolution(self, sweep, t0, dt, dt_out, n, dev, time_ptr, u_ptr, lanes, stream):
         if lanes == "auto":
-            from .autotune import tune_lanes
-            n_fine = math.floor(dt_out / dt + 0.5)
-            lanes, _ = tune_lanes(self, n, n_fine, dt, dt_out, sweep, t0) if n else (0, None)
+            lanes = self._tuned_lanes(sweep, t0, dt, dt_out, n)
         _native.check(_native.lib().ss_time_evolution(
             self._module(dev).handle, sweep.data_ptr(), float(t0), float(dt), float(dt_out), n,
             time_ptr, u_ptr, self._table_ptr(dev), int(lanes), stream), "ss_time_evolution")
@@ -541,26 +544,21 @@ class Simulator:
         stream = torch.cuda.current_stream(dev)
         sweep = np.ascontiguousarray(np.atleast_1d(np.asarray(sweep_parameters, np.float64)))
         lanes = lanes_per_step if lanes_per_step is not None else (self.lanes_per_step or 0)
-        if not 1 <= sweep.size <= _native.SWEEP_INLINE or lanes == "auto":
-            sweep = torch.as_tensor(sweep, device=dev)
+        inline = 1 <= sweep.size <= _native.SWEEP_INLINE
+        if not inline or lanes == "auto":
+            on_device = torch.as_tensor(sweep, device=dev)
+        if lanes == "auto":
+            lanes = self._tuned_lanes(on_device, float(ends[0]), dt, time_step_output, n)
         psi0 = np.ascontiguousarray(np.asarray(state_init, np.complex128).reshape(d))
         ws_bytes = int(_native.lib().ss_evaluate_workspace(n, d))
 
-        def run(time, u, state, spin, ws):
-            """Enqueue time evolution and, with a state, the scan (device addresses)."""
-            if isinstance(sweep, np.ndarray):
-                _native.check(_native.lib().ss_evaluate(
-                    self._module(dev).handle, sweep.ctypes.data, sweep.size, float(ends[0]), dt,
-                    float(time_step_output), n, time, u, self._table_ptr(dev), int(lanes),
-                    psi0.ctypes.data, state, spin, ws, ws_bytes, stream.cuda_stream),
-                    "ss_evaluate")
-                return
-            self._launch_time_evolution(sweep, float(ends[0]), dt, time_step_output, n, dev, time,
-                                        u, lanes, stream.cuda_stream)
-            if state:
-                _native.check(_native.lib().ss_state_scan(
-                    psi0.ctypes.data, u, state, spin, n, d, ws, ws_bytes, stream.cuda_stream),
-                    "ss_state_scan")
+        def run(time, u, state, spin, ws, reader=None):
+            """Enqueue time evolution and state scan (device addresses)."""
+            _native.check(_native.lib().ss_evaluate(
+                self._module(dev).handle, sweep.ctypes.data if inline else on_device.data_ptr(),
+                sweep.size if inline else 0, float(ends[0]), dt, float(time_step_output), n, time, u,
+                self._table_ptr(dev), int(lanes), psi0.ctypes.data, state, spin, ws, ws_bytes,
+                stream.cuda_stream, reader), "ss_evaluate")
 
         # time, U, state and spin one after the other, 256-byte aligned, for
         # results that come back in one copy
@@ -588,22 +586,20 @@ class Simulator:
         if output == "torch":
             run(time.data_ptr(), u.data_ptr(), state.data_ptr(), None, ws.data_ptr())
             return Results(time, u, state, self.spin_calculator)
-        # larger numpy results: time and U go to pinned host memory on a side
-        # stream while the state scan runs, then the states follow
         if n * (d * d + d + 1) * 16 > PINNED_RESULT_BYTES:
             run(time.data_ptr(), u.data_ptr(), state.data_ptr(), None, ws.data_ptr())
             return Results(time.cpu().numpy(), u.cpu().numpy(), state.cpu().numpy(),
                            self.spin_calculator, _device_state=state)
+        # larger numpy results: time and U go to pinned host memory on a side
+        # stream while the states are formed, then those follow
         side = self._copy_stream(dev)
         h_time = torch.empty(time.shape, dtype=time.dtype, pin_memory=True)
         h_u = torch.empty(u.shape, dtype=u.dtype, pin_memory=True)
         h_state = torch.empty((n, d), dtype=u.dtype, pin_memory=True)
-        run(time.data_ptr(), u.data_ptr(), None, None, None)
-        side.wait_stream(stream)
+        run(time.data_ptr(), u.data_ptr(), state.data_ptr(), None, ws.data_ptr(), side.cuda_stream)
         with torch.cuda.stream(side):
             h_time.copy_(time, non_blocking=True)
             h_u.copy_(u, non_blocking=True)
-        self.launch_state_scan(psi0, u, state, ws, stream=stream.cuda_stream)
         h_state.copy_(state, non_blocking=True)
         stream.synchronize()
         side.synchronize()
