@@ -10,7 +10,7 @@ where each control k is an interpolation table (zero-order hold, linear or
 cubic Hermite, exactly the sampler of generate_interpolation_sampler) on a
 time grid, with amplitudes ``c`` (B, K, M) given as a float64 device tensor.
 :meth:`ControlledSimulator.final_state` returns psi(T) (B, d) and is a
-``torch.autograd.Function``: the forward pass runs the batched persistent
+``torch.autograd.Function``: the forward pass runs the batched
 time-evolution launch and the per-simulation state scan and keeps only the
 coarse step operators and states (checkpoints); the backward pass scans the
 costates backward over the coarse operators, then recomputes every fine step

@@ -1,4 +1,4 @@
-"""Batched evaluation: many simulations in one persistent launch.
+"""Batched evaluation: many simulations in one launch.
 
 The reference runs one ``evaluate`` per sweep point (spinsim/__init__.py:993;
 example.py evaluates twice to sweep a bias).  ``BatchPlan`` packs B

@@ -615,7 +615,7 @@ class Simulator:
 
     def evaluate_batch(self, time_start, time_end, time_step_integration, time_step_output,
                        state_init, sweep_parameters, **kw):
-        """Evaluate B simulations (sweep rows) in one persistent launch.
+        """Evaluate B simulations (sweep rows) in one launch.
 
         Any of the times/steps may be per-simulation (B,) arrays and
         ``state_init`` may be (B, d); returns :class:`spinsim_amd.batch.BatchResults`.
