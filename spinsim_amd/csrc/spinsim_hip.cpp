@@ -1762,10 +1762,16 @@ int launch_scan(const char* who, ScanArgs a, int dim, bool reverse, int64_t chun
     a.chunk_rows = l.chunk_rows;
     a.n_chunks = l.chunks;
     const dim3 g(unsigned(l.chunks)), b(kScanThreads);
-    // pass 2 with one row per thread once chunks span several tiles (large,
-    // bandwidth-bound scans: row-contiguous lanes store coalesced); with a
-    // tile's rows per thread when each chunk is one tile (latency-bound)
-    const int rows = l.chunk_rows > kScanTileRows ? 0 : int(l.chunk_rows / kScanThreads);
+    // pass 2 with one row per thread where the scan is bound by its bytes (chunks
+    // of several tiles, or more than 512 of one: row-contiguous lanes store
+    // coalesced), two for spin one backwards; with a tile's rows per thread where
+    // latency bounds it.  2.05e6 rows in simulations of 2000, four rows a thread
+    // -> these: spin half 145 -> 89 us, as first columns 106 -> 62 and 141 -> 72,
+    // backwards 117 -> 87, spin one 290 -> 231 and 251 -> 232; at 5.3e5 rows 52 ->
+    // 38, 41 -> 30, 46 -> 33, 43 -> 37, 89 -> 78 and 81 -> 79, while at 3e5 spin
+    // half backwards (37 against 35) and spin one (65 against 60) were slower
+    const bool many = l.chunk_rows == kScanTileRows && l.chunks > 512;
+    const int rows = many || l.chunk_rows > kScanTileRows ? 0 : int(l.chunk_rows / kScanThreads);
     if (dim == 2 && !reverse && a.u_layout != SS_U_FULL) {
         // special unitary operators: maps composed and moved as first
         // columns.  Pass 1 over wide chunks reads 64 bytes of rows per lane
@@ -1787,6 +1793,8 @@ int launch_scan(const char* who, ScanArgs a, int dim, bool reverse, int64_t chun
         launch_scan_passes<3, false, false>(a, rows, g, b, s);
     } else if (dim == 2) {
         launch_scan_passes<2, true, false>(a, rows, g, b, s);
+    } else if (many) {
+        launch_scan_passes<3, true, false, kScanRows, 2>(a, g, b, s);
     } else {
         launch_scan_passes<3, true, false>(a, rows, g, b, s);
     }
