@@ -39,6 +39,8 @@
 // splitting is what the caller asked for and is carried out.
 #define SS_CONVERGED_HYPER 12
 #define SS_DIRECT_EXPO (SS_EXPO == 0 || SS_HYPER >= SS_CONVERGED_HYPER)
+// Spin one whose steps may be rotations (SS_IS_ROTATION).
+#define SS_SPIN_ONE_ROTATIONS (SS_DIM == 3 && SS_LIE == 4 && SS_PREC == 0 && SS_DIRECT_EXPO)
 
 // sin and cos of x.  The Lie-Trotter generators are scaled by 4^-hypercubes,
 // so their angles are tiny; there the Taylor series to x^9 / x^10 is exact to
@@ -177,7 +179,7 @@ static __device__ __forceinline__ void ss_square_hypercubes(ss_cd a[SS_D][SS_D])
 #endif
 
 // ---- matrix exponentials of -i g.J ----------------------------------------
-#if SS_DIM == 2 && SS_DIRECT_EXPO
+#if (SS_DIM == 2 && SS_DIRECT_EXPO) || SS_SPIN_ONE_ROTATIONS
 // matrix_exponential_analytic, spinsim/__init__.py:1617-1641:
 // exp(-i g.sigma/2) = cos(r/2) I - i (sin(r/2)/r) g.sigma, r2 = r^2 = |g|^2, as
 // the first column (b0, b1) of its residual, exp - I.
@@ -210,6 +212,8 @@ static __device__ __forceinline__ void ss_expo_su2_m1(const double g[SS_FIELD_LE
     b0 = ss_c(c, -z * sr);
     b1 = ss_c(y * sr, -x * sr);
 }
+#endif
+#if SS_DIM == 2 && SS_DIRECT_EXPO
 #elif SS_DIM == 2
 // matrix_exponential_lie_trotter (spin half), spinsim/__init__.py:1643-1673:
 // the first column (b0, b1) of its residual.
@@ -705,7 +709,7 @@ static __device__ __forceinline__ void ss_append(const double g[SS_FIELD_LEN], s
 }
 #endif
 
-#if SS_DIM == 2
+#if SS_DIM == 2 || SS_SPIN_ONE_ROTATIONS
 // Spin-half step operators are special unitary, [[p, -conj q], [q, conj p]],
 // and so are their products, so a chunk's operator is accumulated as its first
 // column: with U = I + a, a's column (p, q) and the step's residual B = E - I,
@@ -776,6 +780,7 @@ static __device__ __forceinline__ void ss_append_su2(const double g[SS_FIELD_LEN
 }
 #endif
 
+#if SS_DIM == 2
 static __device__ __forceinline__ void ss_su2_expand(ss_cd p, ss_cd q, ss_cd u[2][2])
 {
     p.x += 1.0;
@@ -784,6 +789,34 @@ static __device__ __forceinline__ void ss_su2_expand(ss_cd p, ss_cd q, ss_cd u[2
     u[0][1] = ss_c(-q.x, q.y);
     u[1][1] = ss_conj(p);
 }
+#else
+// The rotation of spin one that the spin-half operator [[p, -conj q], [q, conj p]]
+// stands for: its symmetric square.
+static __device__ __forceinline__ void ss_su2_expand(ss_cd p, ss_cd q, ss_cd u[3][3])
+{
+    p.x += 1.0;
+    const double root2 = 1.4142135623730951;
+    const ss_cd pq = ss_scale(ss_mul(p, q), root2);            // sqrt 2 p q
+    const ss_cd rq = ss_scale(ss_mul(ss_conj(p), q), root2);   // sqrt 2 conj(p) q
+    u[0][0] = ss_mul(p, p);
+    u[1][0] = pq;
+    u[2][0] = ss_mul(q, q);
+    u[0][1] = ss_c(-rq.x, rq.y);
+    u[1][1] = ss_c(fma(p.x, p.x, p.y * p.y) - fma(q.x, q.x, q.y * q.y), 0.0);
+    u[2][1] = rq;
+    u[0][2] = ss_conj(u[2][0]);
+    u[1][2] = ss_c(-pq.x, pq.y);
+    u[2][2] = ss_conj(u[0][0]);
+}
+
+// Whether a sample's quadratic shift is known to be zero when the kernel is
+// compiled (the callback leaves the zero it was given, or sets one): the step is
+// then a rotation, and a chunk's operator is accumulated as the spin-half one
+// (about 130 instructions a step in place of 400).  The same for every step, so
+// the other accumulator is compiled out.  1024 simulations of 1e5 steps with two
+// control fields: 1.44 -> 0.69 ms, 216 registers -> 166 (three waves a SIMD).
+#define SS_IS_ROTATION(f) (__builtin_constant_p((f)[3]) && (f)[3] == 0.0)
+#endif
 #endif
 
 #if SS_PREC != 0
@@ -1177,6 +1210,10 @@ static __device__ __forceinline__ void ss_integrate(ss_cd u[SS_D][SS_D], int j0,
 #pragma unroll
     for (int r = 0; r < 3; ++r) su_a[r][0] = su_a[r][1] = ss_c(0.0, 0.0);
 #define SS_APPEND(g) ss_append(g, su_a)
+#if SS_SPIN_ONE_ROTATIONS
+    ss_cd su_p = ss_c(0.0, 0.0), su_q = ss_c(0.0, 0.0);
+    int kind = 0;
+#endif
 #else
 #define SS_APPEND(g) ss_append(g, u)
 #endif
@@ -1207,7 +1244,18 @@ static __device__ __forceinline__ void ss_integrate(ss_cd u[SS_D][SS_D], int j0,
             ss_frame(fa, rot, wa.w);
 #pragma unroll
             for (int k = 0; k < SS_FIELD_LEN; ++k) g[k] = dt * fa[k];
+#if SS_SPIN_ONE_ROTATIONS
+            if (SS_IS_ROTATION(fa)) {
+                ss_append_su2(g, su_p, su_q);
+                if ((j & (SS_SU2_BLOCK - 1)) == SS_SU2_BLOCK - 1) ss_su2_normalise(su_p, su_q);
+                kind = 1;
+            } else {
+                SS_APPEND(g);
+                kind = 2;
+            }
+#else
             SS_APPEND(g);
+#endif
 #else
             double fb[SS_FIELD_LEN];
             ss_call_field(wa.t, sweep, fa, ctx);
@@ -1231,8 +1279,21 @@ static __device__ __forceinline__ void ss_integrate(ss_cd u[SS_D][SS_D], int j0,
                 g2[k] = dt * fb[k] / 2;
             }
 #endif
+#if SS_SPIN_ONE_ROTATIONS
+            if (SS_IS_ROTATION(fa) && SS_IS_ROTATION(fb)) {
+                ss_append_su2(g, su_p, su_q);
+                ss_append_su2(g2, su_p, su_q);
+                if ((j & (SS_SU2_BLOCK - 1)) == SS_SU2_BLOCK - 1) ss_su2_normalise(su_p, su_q);
+                kind = 1;
+            } else {
+                SS_APPEND(g);
+                SS_APPEND(g2);
+                kind = 2;
+            }
+#else
             SS_APPEND(g);
             SS_APPEND(g2);
+#endif
 #endif
             tf += dt;
             ss_wind_advance(wa, tf + off_a, tc, step, frot, dt);
@@ -1249,6 +1310,13 @@ static __device__ __forceinline__ void ss_integrate(ss_cd u[SS_D][SS_D], int j0,
 #elif SS_DIM == 2
     ss_su2_expand(su_p, su_q, u);
 #elif SS_DIRECT_EXPO
+#if SS_SPIN_ONE_ROTATIONS
+    if (kind == 1) {
+        ss_su2_normalise(su_p, su_q);
+        ss_su2_expand(su_p, su_q, u);
+        return;
+    }
+#endif
     ss_su3_expand(su_a, u);
 #endif
 #undef SS_APPEND
