@@ -2127,10 +2127,66 @@ static __device__ __forceinline__ void ss_flush_moments(const ss_adjoint_args& a
     *idx = -1;
 }
 
-// dL/d(lab-frame field) at one sample -> control gradients: moment sums when
-// the control's table has its interval holding t cached (ss_ctx::line, set by
-// the field's own sample at t or a neighbouring one), else weights looked up
-// at t and added to the knots.
+// The cached interval of table `table` (a uniform index: the copy is a uniform
+// branch per line, no dynamic register index); inv_h is NaN when there is none.
+static __device__ __forceinline__ void ss_cached_interval(const ss_ctx* ctx, int table, double* t0, double* inv_h,
+                                                          long long* idx)
+{
+    *t0 = 0.0;
+    *inv_h = __builtin_nan("");
+    *idx = -1;
+#pragma unroll
+    for (int k = 0; k < SS_INTERP_LINES; ++k)
+        if (table == k) {
+            *t0 = ctx->line[k].t0;
+            *inv_h = ctx->line[k].inv_h;
+            *idx = ctx->line[k].idx;
+        }
+}
+
+// Add M_0..M_3 of samples in interval idx to control c's moment sums: LDS adds
+// without return (ds_add_f64) to the lane's own slots, so no read sits on the
+// samples' dependency chain.
+static __device__ __forceinline__ void ss_add_moments(const ss_adjoint_args& a, const ss_ctx* ctx, int c, long long idx,
+                                                      const double mom[4], double* win, long long base_c,
+                                                      double* grad_row, long long mo_idx[SS_ADJ_CONTROLS])
+{
+    long long& mi = mo_idx[c < SS_ADJ_CONTROLS ? c : 0];
+    if (idx != mi) {
+        ss_flush_moments(a, ctx, c, &mi, win, base_c, grad_row);
+        mi = idx;
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+        __hip_atomic_fetch_add(ss_moment_slot(win, c, m), mom[m], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// dL/d(lab-frame field) at one sample, times control c's scale -> its gradient:
+// moment sums when the control's table has its interval holding t cached
+// (ss_ctx::line, set by the field's own sample at t or a neighbouring one), else
+// weights looked up at t and added to the knots.
+static __device__ __forceinline__ void ss_scatter_control(const ss_adjoint_args& a, const ss_ctx* ctx, int c, double t,
+                                                          double v, double t0, double inv_h, long long idx,
+                                                          double* win, long long base_c, double* grad_row,
+                                                          long long mo_idx[SS_ADJ_CONTROLS])
+{
+    const double p = (t - t0) * inv_h;
+    if (c < SS_ADJ_CONTROLS && p >= 0.0 && p <= 1.0) {
+        const double vp = v * p, vp2 = vp * p;
+        const double mom[4] = {v, vp, vp2, vp2 * p};
+        ss_add_moments(a, ctx, c, idx, mom, win, base_c, grad_row, mo_idx);
+        return;
+    }
+    if (v == 0.0) return;
+    const int table = a.controls[c].table;
+    long long first;
+    double w[4];
+    ss_interp_weights(&ctx->tables[table], t, &first, w);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[k] *= v;
+    ss_scatter_knots(a, c, first, w, ctx->tables[table].size, win, base_c, grad_row);
+}
+
 static __device__ __forceinline__ void ss_scatter_sample(const ss_adjoint_args& a, const ss_ctx* ctx, double t,
                                                          const double dfield[4], double* win,
                                                          const long long base[SS_MAX_CONTROLS], double* grad_row,
@@ -2140,44 +2196,41 @@ static __device__ __forceinline__ void ss_scatter_sample(const ss_adjoint_args& 
     for (int c = 0; c < SS_MAX_CONTROLS; ++c) {
         if (c >= a.n_controls) break;
         const ss_control ct = a.controls[c];
-        const double v = ct.scale * dfield[ct.axis];
-        if (c < SS_ADJ_CONTROLS && ct.table < SS_INTERP_LINES) {
-            // the cached interval of table ct.table (a uniform index: the
-            // copy is a uniform branch per line, no dynamic register index)
-            double t0 = 0.0, inv_h = __builtin_nan("");
-            long long idx = -1;
+        double t0, inv_h;
+        long long idx;
+        ss_cached_interval(ctx, ct.table, &t0, &inv_h, &idx);
+        ss_scatter_control(a, ctx, c, t, ct.scale * dfield[ct.axis], t0, inv_h, idx, win, base[c], grad_row, mo_idx);
+    }
+}
+
+// Both samples of a step: where a control's cached interval holds both, as nearly
+// always, their moments are summed first: half the LDS adds and one test for the
+// two (backward pass of 1024 simulations of 1e5 steps with two cubic controls:
+// 1.98 -> 1.92 ms).
+static __device__ __forceinline__ void ss_scatter_pair(const ss_adjoint_args& a, const ss_ctx* ctx, double ta,
+                                                       const double da[4], double tb, const double db[4], double* win,
+                                                       const long long base[SS_MAX_CONTROLS], double* grad_row,
+                                                       long long mo_idx[SS_ADJ_CONTROLS])
+{
 #pragma unroll
-            for (int k = 0; k < SS_INTERP_LINES; ++k)
-                if (ct.table == k) {
-                    t0 = ctx->line[k].t0;
-                    inv_h = ctx->line[k].inv_h;
-                    idx = ctx->line[k].idx;
-                }
-            const double p = (t - t0) * inv_h;
-            if (p >= 0.0 && p <= 1.0) {
-                long long& mi = mo_idx[c < SS_ADJ_CONTROLS ? c : 0];
-                if (idx != mi) {
-                    ss_flush_moments(a, ctx, c, &mi, win, base[c], grad_row);
-                    mi = idx;
-                }
-                // LDS adds without return (ds_add_f64): the lane's own slots,
-                // so no read sits on the sample's dependency chain
-                const double vp = v * p, vp2 = vp * p;
-                __hip_atomic_fetch_add(ss_moment_slot(win, c, 0), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(ss_moment_slot(win, c, 1), vp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(ss_moment_slot(win, c, 2), vp2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(ss_moment_slot(win, c, 3), vp2 * p, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-                continue;
-            }
+    for (int c = 0; c < SS_MAX_CONTROLS; ++c) {
+        if (c >= a.n_controls) break;
+        const ss_control ct = a.controls[c];
+        const double va = ct.scale * da[ct.axis], vb = ct.scale * db[ct.axis];
+        double t0, inv_h;
+        long long idx;
+        ss_cached_interval(ctx, ct.table, &t0, &inv_h, &idx);
+        const double pa = (ta - t0) * inv_h, pb = (tb - t0) * inv_h;
+        // (without an interval both are NaN)
+        if (c < SS_ADJ_CONTROLS && fmin(pa, pb) >= 0.0 && fmax(pa, pb) <= 1.0) {
+            const double a1 = va * pa, b1 = vb * pb, a2 = a1 * pa, b2 = b1 * pb;
+            const double mom[4] = {va + vb, a1 + b1, a2 + b2, fma(a2, pa, b2 * pb)};
+            ss_add_moments(a, ctx, c, idx, mom, win, base[c], grad_row, mo_idx);
+            continue;
         }
-        if (v == 0.0) continue;
-        long long first;
-        double w[4];
-        ss_interp_weights(&ctx->tables[ct.table], t, &first, w);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) w[k] *= v;
-        ss_scatter_knots(a, c, first, w, ctx->tables[ct.table].size, win, base[c], grad_row);
+#pragma unroll 1
+        for (int k = 0; k < 2; ++k)
+            ss_scatter_control(a, ctx, c, k ? tb : ta, k ? vb : va, t0, inv_h, idx, win, base[c], grad_row, mo_idx);
     }
 }
 
@@ -2407,10 +2460,10 @@ ss_batch_adjoint_kernel(ss_adjoint_args a)
             dz_mid += tra * (dfa[0] * fa[1] - dfa[1] * fa[0]) - dfa[2] +
                       trb * (dfb[0] * fb[1] - dfb[1] * fb[0]) - dfb[2];
 #endif
+        double lab_b[4];
         ss_unframe(dfa, wa_w, lab);
-        ss_scatter_sample(a, &ctx, wa.t, lab, win, base, grad_row, mo);
-        ss_unframe(dfb, wb_w, lab);
-        ss_scatter_sample(a, &ctx, wb.t, lab, win, base, grad_row, mo);
+        ss_unframe(dfb, wb_w, lab_b);
+        ss_scatter_pair(a, &ctx, wa.t, lab, wb.t, lab_b, win, base, grad_row, mo);
 #endif
     }
 #if SS_ROT
