@@ -1486,9 +1486,9 @@ static __device__ __forceinline__ const double* ss_te_sweep(const ss_te_args& a)
 // operator on the first lane of each group of `lanes` (the identity on rows
 // from `end` on); the wave's rows start at `first`.
 // A launch and a read of the operators less than a scan of the stored ones
-// (integrator and states together, without spin): 40 spin-half rows of 10 steps
-// 12.6 -> 8.7 us, 20,000 rows 16.9 -> 14.9, 200,000 rows of 5 33.6 -> 25.2;
-// spin one 21.3 -> 13.2, 28.7 -> 27.8 and 64.3 -> 57.8.
+// (integrator and states together, without spin, with the wave scans of ss_wave_scan):
+// 40 spin-half rows of 10 steps 12.6 -> 8.6 us, 20,000 rows 16.9 -> 13.3, 200,000
+// rows of 5 33.6 -> 24.0; spin one 21.3 -> 12.8, 28.7 -> 23.5 and 64.3 -> 53.2.
 static __device__ __forceinline__ void ss_scan_block(ss_cd u[SS_D][SS_D], int lanes, long long first, long long end,
                                                      double* prefix, double* block_total)
 {

@@ -145,10 +145,11 @@ __global__ void __launch_bounds__(256) spin_kernel(const double* state, double* 
     ss_store_spin<D>(s, spin, i);
 }
 
-// ---- state scan of one simulation: three passes ---------------------------
-// The latency-bound case (1e5 rows take ~25 us): per-lane prefix products
-// within 256-lane workgroups, one workgroup scanning the block totals into
-// block carries, and a pass applying prefix x carry to psi0 per row.
+// ---- state scan of one simulation -----------------------------------------
+// Of stored operators (latency-bound: 1e5 spin-one rows take 16 us): per-lane
+// prefix products within 256-lane workgroups and a pass that forms each
+// workgroup's carry from the totals before it and applies prefix x carry to psi0
+// per row; beyond kFusedScanBlocks one workgroup scans the totals in between.
 
 constexpr int kSingleScanChunk = 2;   // matrices per lane
 constexpr int kSingleScanBlock = 256;
