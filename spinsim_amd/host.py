@@ -132,11 +132,14 @@ def module_source(field_src, dim, method, expo, rotating, number_of_squares, has
             f"#define SS_EXPO {expo}\n#define SS_ROT {1 if rotating else 0}\n"
             f"#define SS_HYPER {hyper}\n#define SS_CTX {1 if has_context else 0}\n"
             f"#define SS_PREC {precision}\n")
-    # the callback's sin, cos and exp: the table-driven float64 functions, or with
-    # precision fp32 the float32 ones (ss_prelude.h), as on the GPU
+    # the callback's sin and cos: the table-driven float64 functions, or with
+    # precision fp32 float32 ones with exp as well (ss_prelude.h), as on the GPU;
+    # exp stays the library's otherwise (within an ulp of the GPU's), so that a
+    # callback may call it as std::exp
+    functions = ("sin", "cos", "exp") if precision == 3 else ("sin", "cos")
     bits = 32 if precision == 3 else 64
-    on = "".join(f"#define {f}(x) ss_{f}{bits}(x)\n" for f in ("sin", "cos", "exp"))
-    off = "#undef sin\n#undef cos\n#undef exp\n"
+    on = "".join(f"#define {f}(x) ss_{f}{bits}(x)\n" for f in functions)
+    off = "".join(f"#undef {f}\n" for f in functions)
     return (head + '#include "host/ss_host_prelude.h"\n#include "device/ss_args.h"\n'
             '#include "device/ss_complex.h"\n#include "device/ss_prelude.h"\n'
             + on + '#line 1 "get_field"\n' + field_src + "\n" + off +
