@@ -343,6 +343,16 @@ static __device__ __forceinline__ void ss_su3_orthonormal(ss_cd b[3][3])
     for (int r = 0; r < 3; ++r) b[r][r].x -= 1.0;
 }
 
+#if SS_LIE == 8
+// det G of ss_expo_su3_m1's entries; n0, n1, nv the squares of l0, l1, v.
+static __device__ __forceinline__ double ss_su3_det8(double d0, double d1, double d2, double n0, double n1, double nv,
+                                                     ss_cd l0, ss_cd l1, ss_cd v)
+{
+    const ss_cd ll = ss_mul(l0, l1);
+    return d0 * d1 * d2 - d0 * n1 - d1 * nv - d2 * n0 + 2.0 * (ll.x * v.x + ll.y * v.y);
+}
+#endif
+
 // b = exp(-i g.J) - I.
 static __device__ __forceinline__ void ss_expo_su3_m1(const double g[SS_FIELD_LEN], ss_cd b[3][3])
 {
@@ -357,14 +367,14 @@ static __device__ __forceinline__ void ss_expo_su3_m1(const double g[SS_FIELD_LE
     ss_cd v = ss_c(g[4], g[5]);
     double n0 = l0.x * l0.x + l0.y * l0.y, n1 = l1.x * l1.x + l1.y * l1.y, nv = v.x * v.x + v.y * v.y;
     double p = d0 * d0 + d2 * (d0 + d2) + n0 + n1 + nv;
-    const ss_cd ll = ss_mul(l0, l1);
-    double q = d0 * d1 * d2 - d0 * n1 - d1 * nv - d2 * n0 + 2.0 * (ll.x * v.x + ll.y * v.y);
+#define SS_SU3_DET() ss_su3_det8(d0, d1, d2, n0, n1, nv, l0, l1, v)
 #else
     ss_cd l = ss_c(g[0] * SS_INV_SQRT2, g[1] * SS_INV_SQRT2);
     double n = l.x * l.x + l.y * l.y;
     double p = d0 * d0 + d2 * (d0 + d2) + 2.0 * n;
-    double q = d1 * fma(d0, d2, n);
+#define SS_SU3_DET() (d1 * fma(d0, d2, n))
 #endif
+    double q = SS_SU3_DET();
     int squares = 0;
     ss_su3_coef k;
     if (p <= SS_SU3_P_SMALL) {
@@ -379,7 +389,6 @@ static __device__ __forceinline__ void ss_expo_su3_m1(const double g[SS_FIELD_LE
             d1 *= f;
             d2 *= f;
             p *= f2;
-            q = q * f * f2;
 #if SS_LIE == 8
             l0 = ss_scale(l0, f);
             l1 = ss_scale(l1, f);
@@ -391,9 +400,12 @@ static __device__ __forceinline__ void ss_expo_su3_m1(const double g[SS_FIELD_LE
             l = ss_scale(l, f);
             n *= f2;
 #endif
+            // (of the scaled entries: the cubic overflows where p does not)
+            q = SS_SU3_DET();
         }
         k = ss_su3_series(p, q);
     }
+#undef SS_SU3_DET
 #if SS_LIE == 8
     const double s0 = fma(d0, d0, n0 + nv), s1 = fma(d1, d1, n0 + n1), s2 = fma(d2, d2, n1 + nv);
     // off-diagonal entries of G^2, e.g. (1, 0): l0 (d0 + d1) + conj(l1) v

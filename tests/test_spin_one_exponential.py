@@ -55,3 +55,20 @@ def test_non_finite_field(device, value):
     sim = ss.Simulator(src, ss.SpinQuantumNumber.ONE, device=device)
     u = sim.evaluate(0.0, 1.5, 1.0, 1.0, [1, 0, 0], [value]).time_evolution
     assert not np.isfinite(u).any()
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("method", METHODS)
+@pytest.mark.parametrize("size", [1e100, 1e103, 1e110, 1e140, 1e152])
+def test_fields_whose_cube_overflows(device, method, size):
+    """The generator's determinant is cubic in the field; the operator stays
+    unitary as long as the squares are finite."""
+    n = 8 if method is METHODS[1] else 4
+    src = ("__device__ void get_field(double t, const double* s, double* f)\n"
+           "{ for (int k = 0; k < %d; ++k) f[k] = s[k]; }" % n)
+    sim = ss.Simulator(src, ss.SpinQuantumNumber.ONE, device=device, exponentiation_method=method,
+                       use_rotating_frame=False, integration_method=ss.IntegrationMethod.EULER)
+    g = size * np.array([1.0, 0.3, 0.7, 0.5, 0.2, 0.1, -0.3, 0.4][:n])
+    u = sim.evaluate(0.0, 1.5, 1.0, 1.0, [1, 0, 0], list(g)).time_evolution[0]
+    # (each square past the first eight is followed by a normalisation)
+    assert np.abs(u.conj().T @ u - np.eye(3)).max() <= 64 * EPS
