@@ -286,7 +286,8 @@ int ss_batch_final_state(const double *psi0, const double *u, const double *stat
  * (n_sims, grad_stride) and *status are cleared by the call; status bit 1 is
  * set if a step's generator was too large for the derivative series, status
  * bit 4 if a control's axis is outside the module's SS_ADJ_AXES (its rows
- * then add nothing).
+ * then add nothing), status bit 8 if the compiled kernel took a callback's
+ * quadratic shift for a constant zero in some steps of a row only.
  * workspace NULL: contributions are summed with float64 atomics, so the
  * rounding of a gradient entry can differ from run to run (sums of the same
  * terms in another order).  workspace of ss_batch_adjoint_workspace(total,

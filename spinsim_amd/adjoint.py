@@ -228,6 +228,9 @@ class ControlledSimulator:
         if flags & 4:
             raise RuntimeError("ss_batch_adjoint: a control's axis is not among those the "
                                "module was compiled for (SS_ADJ_AXES)")
+        if flags & 8:
+            raise RuntimeError("ss_batch_adjoint: the compiler takes the quadratic shift for zero in "
+                               "some steps only; set it from a sweep parameter instead")
         return grad
 
 

@@ -94,7 +94,9 @@ struct ss_adjoint_args {
     const double* costate;       // (total, d)
     double* grad;                // (B, grad_stride), accumulated with atomics
     int* status;                 // bit 1: a step too large for the series;
-                                 // bit 2: a sample outside the window (deterministic mode)
+                                 // bit 2: a sample outside the window (deterministic mode);
+                                 // bit 4: a control's axis outside SS_ADJ_AXES;
+                                 // bit 8: steps of both kinds in one row
     double* partial;             // deterministic mode: (total, n_controls, SS_ADJ_WINDOW)
                                  // window contents per row, or null (atomics)
     long long* window_base;      // deterministic mode: (total, n_controls) window starts

@@ -824,8 +824,9 @@ static __device__ __forceinline__ void ss_su2_expand(ss_cd p, ss_cd q, ss_cd u[3
 // Whether a sample's quadratic shift is known to be zero when the kernel is
 // compiled (the callback leaves the zero it was given, or sets one): the step is
 // then a rotation, and a chunk's operator is accumulated as the spin-half one
-// (about 130 instructions a step in place of 400).  The same for every step, so
-// the other accumulator is compiled out.  1024 simulations of 1e5 steps with two
+// (about 130 instructions a step in place of 400).  The same for every step (the
+// builtin is convergent: its branch is not copied onto the paths of a callback
+// that sets the shift on some of them), so the other accumulator is compiled out.  1024 simulations of 1e5 steps with two
 // control fields: 1.44 -> 0.69 ms, 216 registers -> 166 (three waves a SIMD).
 #define SS_IS_ROTATION(f) (__builtin_constant_p((f)[3]) && (f)[3] == 0.0)
 #endif
@@ -1224,7 +1225,7 @@ static __device__ __forceinline__ void ss_integrate(ss_cd u[SS_D][SS_D], int j0,
 #define SS_APPEND(g) ss_append(g, su_a)
 #if SS_SPIN_ONE_ROTATIONS
     ss_cd su_p = ss_c(0.0, 0.0), su_q = ss_c(0.0, 0.0);
-    int kind = 0;
+    bool rotated = false, general = false;  // which accumulators hold steps
 #endif
 #else
 #define SS_APPEND(g) ss_append(g, u)
@@ -1260,10 +1261,10 @@ static __device__ __forceinline__ void ss_integrate(ss_cd u[SS_D][SS_D], int j0,
             if (SS_IS_ROTATION(fa)) {
                 ss_append_su2(g, su_p, su_q);
                 if ((j & (SS_SU2_BLOCK - 1)) == SS_SU2_BLOCK - 1) ss_su2_normalise(su_p, su_q);
-                kind = 1;
+                rotated = true;
             } else {
                 SS_APPEND(g);
-                kind = 2;
+                general = true;
             }
 #else
             SS_APPEND(g);
@@ -1296,11 +1297,11 @@ static __device__ __forceinline__ void ss_integrate(ss_cd u[SS_D][SS_D], int j0,
                 ss_append_su2(g, su_p, su_q);
                 ss_append_su2(g2, su_p, su_q);
                 if ((j & (SS_SU2_BLOCK - 1)) == SS_SU2_BLOCK - 1) ss_su2_normalise(su_p, su_q);
-                kind = 1;
+                rotated = true;
             } else {
                 SS_APPEND(g);
                 SS_APPEND(g2);
-                kind = 2;
+                general = true;
             }
 #else
             SS_APPEND(g);
@@ -1323,7 +1324,10 @@ static __device__ __forceinline__ void ss_integrate(ss_cd u[SS_D][SS_D], int j0,
     ss_su2_expand(su_p, su_q, u);
 #elif SS_DIRECT_EXPO
 #if SS_SPIN_ONE_ROTATIONS
-    if (kind == 1) {
+    // (one of the two is a constant false; were some steps' shift known to be zero
+    // and others' not, their order would be lost, and the operator is NaN)
+    if (rotated) {
+        if (general) su_p.x = __builtin_nan("");
         ss_su2_normalise(su_p, su_q);
         ss_su2_expand(su_p, su_q, u);
         return;
@@ -2394,6 +2398,7 @@ ss_batch_adjoint_kernel(ss_adjoint_args a)
 #pragma unroll
     for (int k = 0; k < SS_LIE; ++k) m[k] = 0.0;
     ss_grad_dots(lam, psi, 7u, 1.0, m);
+    bool rotated = false, general = false;  // what the steps walked: m, or psi and lam
 #pragma unroll 1
     for (int j = n_fine - 1; j >= 0; --j) {
         if (j < n_fine - 1) {
@@ -2413,8 +2418,13 @@ ss_batch_adjoint_kernel(ss_adjoint_args a)
 #if SS_METHOD == 1
 #pragma unroll
         for (int k = 0; k < SS_FIELD_LEN; ++k) g1[k] = dt * fa[k];
-        if (SS_ADJ_ROTATES(fa)) ss_adjoint_rotate(g1, m, d1, a.status);
-        else ss_adjoint_exp(g1, psi, lam, mask, d1, a.status);
+        if (SS_ADJ_ROTATES(fa)) {
+            ss_adjoint_rotate(g1, m, d1, a.status);
+            rotated = true;
+        } else {
+            ss_adjoint_exp(g1, psi, lam, mask, d1, a.status);
+            general = true;
+        }
 #pragma unroll
         for (int k = 0; k < SS_LIE; ++k) dfa[k] = dt * d1[k];
 #if SS_ROT
@@ -2439,9 +2449,11 @@ ss_batch_adjoint_kernel(ss_adjoint_args a)
         if (SS_ADJ_ROTATES(fa) && SS_ADJ_ROTATES(fb)) {
             ss_adjoint_rotate(g2, m, d2, a.status);
             ss_adjoint_rotate(g1, m, d1, a.status);
+            rotated = true;
         } else {
             ss_adjoint_exp(g2, psi, lam, mask, d2, a.status);
             ss_adjoint_exp(g1, psi, lam, mask, d1, a.status);
+            general = true;
         }
 #pragma unroll
         for (int k = 0; k < SS_LIE; ++k) {
@@ -2457,9 +2469,11 @@ ss_batch_adjoint_kernel(ss_adjoint_args a)
         if (SS_ADJ_ROTATES(fa) && SS_ADJ_ROTATES(fb)) {
             ss_adjoint_rotate(g2, m, d2, a.status);
             ss_adjoint_rotate(g1, m, d1, a.status);
+            rotated = true;
         } else {
             ss_adjoint_exp(g2, psi, lam, mask, d2, a.status);
             ss_adjoint_exp(g1, psi, lam, mask, d1, a.status);
+            general = true;
         }
 #pragma unroll
         for (int k = 0; k < SS_LIE; ++k) {
@@ -2478,6 +2492,8 @@ ss_batch_adjoint_kernel(ss_adjoint_args a)
         ss_scatter_pair(a, &ctx, wa.t, lab, wb.t, lab_b, win, base, grad_row, mo);
 #endif
     }
+    // (one of the two is a constant false, as in ss_integrate; a mixture is refused)
+    if (rotated && general) atomicOr(a.status, 8);
 #if SS_ROT
     if (z_control) {
         const double dmid[4] = {0.0, 0.0, dz_mid, 0.0};
