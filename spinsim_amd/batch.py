@@ -310,7 +310,8 @@ def default_batch_items(total_rows, lanes):
     us at one, 81 at four, 91 at sixteen; 4e5 rows of 10 steps: 36 us at one, 38
     at four; 1.1e8 rows of 20 steps: 9.05 ms at four, 8.94 at eight, 9.01 at
     thirty-two)."""
-    waves = -(-int(total_rows) // (64 // lanes))
+    # (lanes above 64 are refused by the launch)
+    waves = -(-int(total_rows) // max(1, 64 // lanes))
     return max(1, min(4, waves // 6000), min(8, waves // 100000))
 
 
