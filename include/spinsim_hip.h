@@ -168,9 +168,8 @@ int ss_module_info(const ss_module *m, int *vgprs, int *sgprs, int *scratch_byte
  * dt_out), taken out of the rotating frame.  `dt` is the integration step as
  * evaluate() re-derives it.  sweep: device array read by get_field; tables:
  * device ss_table array or NULL.  lanes_per_step in 1..64: that many lanes
- * share one coarse step; 0 (the default): the lanes ss_default_lanes gives for
- * the module and the device, or -3 (spin half) or -2 (spin one) in the float32
- * modes; -k (1..64): k waves per SIMD, with rows dealt in
+ * share one coarse step; 0 (the default): what ss_default_launch gives for
+ * the module and the device; -k (1..64): k waves per SIMD, with rows dealt in
  * phases of decreasing item length (lanes per step) so the waves finish
  * together.  u_out: n_coarse*dim*dim complex128. */
 int ss_time_evolution(const ss_module *m, const double *sweep, double t0, double dt,
@@ -197,6 +196,15 @@ size_t ss_evaluate_workspace(int64_t n, int dim);
  * 1 for invalid arguments).  (No reference counterpart: a launch-planning
  * query.) */
 int ss_default_lanes(int64_t n_rows, int n_fine, int64_t cus, int64_t resident);
+/* How a module's step operators are computed. */
+#define SS_STEPS_DIRECT 1  /* float64 */
+#define SS_STEPS_FLOAT32 2 /* the float32 modes */
+/* lanes_per_step that ss_time_evolution takes for 0, for a module of which
+ * `resident` workgroups of the kernel of fixed lanes and `resident_phased` of
+ * the phased one fit a CU (host only; 1 for invalid arguments): ss_default_lanes,
+ * or -k.  (No reference counterpart: a launch-planning query.) */
+int ss_default_launch(int dim, int steps, int64_t n_rows, int n_fine, int64_t cus,
+                      int64_t resident, int64_t resident_phased);
 /* The phase table a phased ss_time_evolution launch on `waves` waves uses
  * (host only): *n_phases phases; phase p starts at coarse row first_row[p]
  * and has items[p] items of 64/lanes[p] rows, each row's fine steps split

@@ -50,6 +50,7 @@ SIGNATURES = {
                               c_vp]),
     "ss_batch_scan_workspace": (ctypes.c_size_t, [c_i64, c_int, c_i64]),
     "ss_default_lanes": (c_int, [c_i64, c_int, c_i64, c_i64]),
+    "ss_default_launch": (c_int, [c_int, c_int, c_i64, c_int, c_i64, c_i64, c_i64]),
     "ss_time_evolution_plan": (c_int, [c_i64, c_int, c_i64, c_vp, c_vp, c_vp, c_vp]),
     "ss_batch_state_scan": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_int, c_i64,
                                     c_int, c_vp, ctypes.c_size_t, c_vp]),

@@ -83,9 +83,10 @@ struct ss_module {
     int expo = 0;
     int rotating = 1;
     int device = 0;
-    bool float32 = false;          // float32-bulk step operators
+    int steps = SS_STEPS_DIRECT;   // how the step operators are computed
     long long cus = 0;             // compute units of the device
     long long single_blocks = 0;   // single kernel: workgroups resident per CU
+    long long phased_blocks = 0;   // phased kernel: the same
 };
 
 // ---------------------------------------------------------------------------
@@ -1399,19 +1400,21 @@ int ss_module_load(const void* code, size_t code_size, int dim, int method, int 
     size_t traits_size = 0;
     if (e == hipSuccess && hipModuleGetGlobal(&traits, &traits_size, m->module, "ss_module_traits") != hipSuccess) {
         (void)hipGetLastError();
-        traits_size = 1;
+        traits_size = SS_STEPS_DIRECT;
     }
-    int per_cu = 0, cus = 0;
+    int per_cu = 0, phased_per_cu = 0, cus = 0;
     if (e == hipSuccess) e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m->single, 256, 0);
+    if (e == hipSuccess) e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&phased_per_cu, m->phased, 256, 0);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, m->device);
     if (e != hipSuccess) {
         if (m->module) (void)hipModuleUnload(m->module);
         delete m;
         return fail("ss_module_load: %s", hipGetErrorString(e));
     }
-    m->float32 = traits_size == 2;
+    m->steps = int(traits_size);
     m->cus = std::max(1, cus);
     m->single_blocks = std::max(1, per_cu);
+    m->phased_blocks = std::max(1, phased_per_cu);
     *out = m;
     return 0;
 }
@@ -1467,8 +1470,7 @@ int ss_module_info(const ss_module* m, int* vgprs, int* sgprs, int* scratch_byte
 // (18 sizes of 40 to 3e5 rows and 1 to 100 steps, seven kernels of 0.1 to 1 us
 // a step): the chosen G is 0.8% slower than the best one on average, 11% at
 // worst, where the launch it replaces (phases over the resident waves) was 28%
-// slower on average and up to 5x.  The float32 modes keep that launch: their
-// chunks round in float32, so their results depend on where rows are cut.
+// slower on average and up to 5x.
 static int default_lanes(long long n_coarse, int n_fine, long long cus, long long resident)
 {
     int best = 1;
@@ -1493,6 +1495,23 @@ static int default_lanes(long long n_coarse, int n_fine, long long cus, long lon
         }
     }
     return best;
+}
+
+// lanes_per_step of the default launch.  The float32 modes' chunks round in
+// float32, so their results depend on where rows are cut: they keep phases over
+// three (spin one: two) waves per SIMD, and no more than the kernel has resident
+// -- the waves beyond would start when the others end (138,836 spin-half rows of
+// 7 steps with eight float32 Gaussians a sample, two resident: 59 us on three,
+// 26 on two).  Rows of one step are never cut, and take all the waves that fit
+// (4e6 of a constant field 108 -> 101 us).
+static int default_launch(int dim, int steps, long long n_coarse, int n_fine, long long cus, long long single_blocks,
+                          long long phased_blocks)
+{
+    if (steps == SS_STEPS_FLOAT32) {
+        const long long waves = n_fine == 1 ? phased_blocks : std::min<long long>(dim == 2 ? 3 : 2, phased_blocks);
+        return -int(std::min(waves, 64LL));
+    }
+    return default_lanes(n_coarse, n_fine, cus, single_blocks);
 }
 
 // Phase table of the phased launch (lanes_per_step = -k) on `waves` waves.
@@ -1550,6 +1569,15 @@ int ss_default_lanes(int64_t n_rows, int n_fine, int64_t cus, int64_t resident)
     return default_lanes(n_rows, n_fine, cus, resident);
 }
 
+int ss_default_launch(int dim, int steps, int64_t n_rows, int n_fine, int64_t cus, int64_t resident,
+                      int64_t resident_phased)
+{
+    if ((dim != 2 && dim != 3) || n_rows < 1 || n_fine < 0 || cus < 1 || resident < 1 || resident_phased < 1 ||
+        n_rows > (1LL << 40))
+        return 1;
+    return default_launch(dim, steps, n_rows, n_fine, cus, resident, resident_phased);
+}
+
 int ss_time_evolution_plan(int64_t n_coarse, int n_fine, int64_t waves, int* n_phases, int* lanes,
                            int64_t* first_row, int64_t* items)
 {
@@ -1599,8 +1627,8 @@ static int time_evolution(const char* who, const ss_module* m, const double* swe
     ss_sample_offsets(m->method, dt, &a.off_a, &a.off_b);
     a.n_fine = n_fine;
     if (lanes_per_step == 0)
-        lanes_per_step = m->float32 ? (m->dim == 2 ? -3 : -2)
-                                    : default_lanes(n_coarse, n_fine, m->cus, m->single_blocks);
+        lanes_per_step =
+            default_launch(m->dim, m->steps, n_coarse, n_fine, m->cus, m->single_blocks, m->phased_blocks);
     if (lanes_per_step > 0) {
         const long long groups = 64 / lanes_per_step;
         a.n_phases = 1;
