@@ -1217,7 +1217,7 @@ ScanLayout scan_layout(int64_t n, int dim, int64_t chunk_rows = 0)
 }
 
 std::string build_source(const char* field_src, int dim, int method, int expo, int rotating,
-                         int number_of_squares, int field_has_context, int precision)
+                         int number_of_squares, int field_has_context, int precision, bool far_inline)
 {
     int hyper = (number_of_squares + 1) / 2;  // ceil(squares / 2), :1547
     if (number_of_squares <= 0) hyper = 0;
@@ -1232,6 +1232,7 @@ std::string build_source(const char* field_src, int dim, int method, int expo, i
         if (std::strstr(field_src, "cos") || std::strstr(field_src, "sin")) s += "#define SS_TRIG_LDS 1\n";
         if (std::strstr(field_src, "exp")) s += "#define SS_EXP_LDS 1\n";
     }
+    if (far_inline) s += "#define SS_TRIG_FAR_INLINE 1\n";
     char head[512];
     snprintf(head, sizeof(head),
              "#define SS_DIM %d\n#define SS_LIE %d\n#define SS_METHOD %d\n#define SS_EXPO %d\n"
@@ -1255,6 +1256,50 @@ std::string build_source(const char* field_src, int dim, int method, int expo, i
     s += ss_src_integrator;
     return s;
 }
+
+hiprtcResult compile_source(const std::string& source, std::string* log, std::vector<char>* object)
+{
+    hiprtcProgram prog;
+    hiprtcResult rc = hiprtcCreateProgram(&prog, source.c_str(), "spinsim_field.hip", 0, nullptr, nullptr);
+    if (rc != HIPRTC_SUCCESS) return rc;
+    rc = hiprtcCompileProgram(prog, int(sizeof(kRtcOptions) / sizeof(kRtcOptions[0])), kRtcOptions);
+    size_t size = 0;
+    hiprtcGetProgramLogSize(prog, &size);
+    log->assign(size, '\0');
+    if (size) hiprtcGetProgramLog(prog, &(*log)[0]);
+    size = 0;
+    if (rc == HIPRTC_SUCCESS) rc = hiprtcGetCodeSize(prog, &size);
+    object->resize(size);
+    if (rc == HIPRTC_SUCCESS) rc = hiprtcGetCode(prog, object->data());
+    hiprtcDestroyProgram(&prog);
+    return rc;
+}
+
+// Vector registers of a code object's ss_time_evolution_kernel, from its metadata
+// note (MessagePack maps with sorted keys: each kernel's .vgpr_count follows its
+// .symbol); 0 if there is none.
+int time_evolution_registers(const std::vector<char>& object)
+{
+    const char symbol[] = "ss_time_evolution_kernel.kd", key[] = ".vgpr_count";
+    auto at = std::search(object.begin(), object.end(), symbol, symbol + sizeof(symbol) - 1);
+    // (the name stands in the symbol tables too)
+    for (; at != object.end(); at = std::search(at + 1, object.end(), symbol, symbol + sizeof(symbol) - 1)) {
+        const auto end = object.end() - at > 256 ? at + 256 : object.end();
+        const auto found = std::search(at, end, key, key + sizeof(key) - 1);
+        if (end - found < long(sizeof(key)) + 2) continue;
+        const unsigned char* v = reinterpret_cast<const unsigned char*>(&*found) + sizeof(key) - 1;
+        if (v[0] < 0x80) return v[0];
+        if (v[0] == 0xcc) return v[1];
+        if (v[0] == 0xcd) return v[1] << 8 | v[2];
+    }
+    return 0;
+}
+
+// Registers of ss_time_evolution_kernel beyond which a callback with sin or cos
+// is compiled with SS_TRIG_FAR_INLINE as well, and the form of fewer is kept (the
+// second compilation takes about two seconds).  With one to three of them a sample
+// the kernel takes 107 to 192, and the first form is the faster one or equal.
+constexpr int kManyRegisters = 200;
 
 // Events for the next time-evolution call on this thread (ss_time_evolution_events).
 thread_local hipEvent_t g_te_start = nullptr, g_te_stop = nullptr;
@@ -1345,35 +1390,31 @@ int ss_compile_code(const char* field_src, int dim, int method, int expo, int ro
     if (precision != SS_PRECISION_FP64 && precision != SS_PRECISION_FP32_BULK &&
         precision != SS_PRECISION_FP64_SERIES && precision != SS_PRECISION_FP32)
         return fail("ss_compile_code: bad precision %d", precision);
-    const std::string src = build_source(field_src, dim, method, expo, rotating, number_of_squares,
-                                         field_has_context, precision);
-    hiprtcProgram prog;
-    if (hiprtcCreateProgram(&prog, src.c_str(), "spinsim_field.hip", 0, nullptr, nullptr) !=
-        HIPRTC_SUCCESS)
-        return fail("hiprtcCreateProgram failed");
-    hiprtcResult rc = hiprtcCompileProgram(prog, int(sizeof(kRtcOptions) / sizeof(kRtcOptions[0])), kRtcOptions);
-    size_t log_size = 0;
-    hiprtcGetProgramLogSize(prog, &log_size);
-    std::string text(log_size, '\0');
-    if (log_size) hiprtcGetProgramLog(prog, &text[0]);
+    std::string source = build_source(field_src, dim, method, expo, rotating, number_of_squares, field_has_context,
+                                      precision, false);
+    std::string text;
+    std::vector<char> object;
+    const hiprtcResult rc = compile_source(source, &text, &object);
     if (log) {
         *log = static_cast<char*>(std::malloc(text.size() + 1));
         if (*log) std::memcpy(*log, text.c_str(), text.size() + 1);
     }
-    if (rc != HIPRTC_SUCCESS) {
-        hiprtcDestroyProgram(&prog);
-        return fail("hipRTC could not compile get_field with the integrator: %s\n%s",
-                    hiprtcGetErrorString(rc), text.c_str());
+    if (rc != HIPRTC_SUCCESS)
+        return fail("hipRTC could not compile get_field with the integrator: %s\n%s", hiprtcGetErrorString(rc),
+                    text.c_str());
+    const int registers = time_evolution_registers(object);
+    if (registers > kManyRegisters && (std::strstr(field_src, "cos") || std::strstr(field_src, "sin"))) {
+        source = build_source(field_src, dim, method, expo, rotating, number_of_squares, field_has_context, precision,
+                              true);
+        std::vector<char> other;
+        const bool compiled = compile_source(source, &text, &other) == HIPRTC_SUCCESS;
+        const int fewer = compiled ? time_evolution_registers(other) : 0;
+        if (fewer > 0 && fewer < registers) object.swap(other);
     }
-    size_t n = 0;
-    hiprtcGetCodeSize(prog, &n);
+    const size_t n = object.size();
     void* buf = std::malloc(n);
-    if (!buf) {
-        hiprtcDestroyProgram(&prog);
-        return fail("out of host memory");
-    }
-    hiprtcGetCode(prog, static_cast<char*>(buf));
-    hiprtcDestroyProgram(&prog);
+    if (!buf) return fail("out of host memory");
+    std::memcpy(buf, object.data(), n);
     *code = buf;
     *code_size = n;
     return 0;
