@@ -181,16 +181,22 @@ int ss_time_evolution(const ss_module *m, const double *sweep, double t0, double
  * reused at once; n_sweep 0: sweep is a device array, as there), then, unless state is NULL, ss_state_scan of its operators
  * (psi0 in host memory; spin NULL or (n, 3); a workspace of that call's size).
  * With a workspace of ss_evaluate_workspace bytes the integrator leaves the
- * scan's products itself where its launch has at most 16,384 workgroups, and one
- * pass writes the states (beyond 1024, after one for the carries).  reader:
- * NULL, or a stream that then waits for the operators and times (to copy them
- * while the states are formed). */
+ * scan's products itself where its launch has one lane per coarse step and at
+ * most 16,384 workgroups, or more lanes and at most 1,024 (a phased launch, so
+ * the default one of the float32 modes, never does), and one pass writes the
+ * states (beyond 1024, after one for the carries); other launches need
+ * ss_state_scan_workspace bytes.  reader: NULL, or a stream that then waits for
+ * the operators and times (to copy them while the states are formed). */
 int ss_evaluate(const ss_module *m, const double *sweep, int n_sweep, double t0, double dt,
                 double dt_out, int64_t n_coarse, double *time_out, double *u_out,
                 const ss_table *tables, int lanes_per_step, const double *psi0, double *state,
                 double *spin, void *workspace, size_t workspace_bytes, ss_stream stream,
                 ss_stream reader);
 size_t ss_evaluate_workspace(int64_t n, int dim);
+/* The bytes that an ss_evaluate call of these arguments makes use of: a product
+ * per row only where its launch leaves them. */
+size_t ss_module_evaluate_workspace(const ss_module *m, int64_t n, double dt, double dt_out,
+                                    int lanes_per_step);
 /* Lanes per coarse step of the default launch for n_rows rows of n_fine steps
  * on `cus` compute units that hold `resident` workgroups each (host only; 1..64,
  * 1 for invalid arguments).  (No reference counterpart: a launch-planning

@@ -45,6 +45,7 @@ SIGNATURES = {
                                         c_i64, c_vp, c_vp, c_vp, c_vp, c_int, c_int, c_int,
                                         c_int, c_vp]),
     "ss_evaluate_workspace": (ctypes.c_size_t, [c_i64, c_int]),
+    "ss_module_evaluate_workspace": (ctypes.c_size_t, [c_vp, c_i64, c_dbl, c_dbl, c_int]),
     "ss_state_scan_workspace": (ctypes.c_size_t, [c_i64, c_int]),
     "ss_state_scan": (c_int, [c_vp, c_vp, c_vp, c_vp, c_i64, c_int, c_vp, ctypes.c_size_t,
                               c_vp]),

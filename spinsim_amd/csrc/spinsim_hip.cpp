@@ -1636,6 +1636,20 @@ int ss_time_evolution_plan(int64_t n_coarse, int n_fine, int64_t waves, int* n_p
     return 0;
 }
 
+// Workgroups of a launch of `lanes` lanes per coarse step.
+static long long lane_blocks(int lanes, long long n_coarse)
+{
+    const long long groups = 64 / lanes;
+    return ((n_coarse + groups - 1) / groups + 3) / 4;
+}
+
+// Whether the integrator of ss_evaluate leaves the scan's products at these lanes
+// per coarse step (a phased launch has no workgroups of consecutive rows).
+static bool leaves_products(int lanes, long long n_coarse)
+{
+    return lanes > 0 && lane_blocks(lanes, n_coarse) <= (lanes == 1 ? kEvaluateBlocks : kFusedScanBlocks);
+}
+
 // ss_time_evolution with the sweep parameters in a device array, or (sweep null)
 // n_inline of them in host memory, which go into the kernel arguments.
 static int time_evolution(const char* who, const ss_module* m, const double* sweep, const double* sweep_host,
@@ -1682,7 +1696,7 @@ static int time_evolution(const char* who, const ss_module* m, const double* swe
     }
     const long long blocks = (a.waves + 3) / 4;
     if (blocks > 2147483647LL) return fail("%s: grid too large", who);
-    if (scan && lanes_per_step > 0 && blocks <= (lanes_per_step == 1 ? kEvaluateBlocks : kFusedScanBlocks)) {
+    if (scan && leaves_products(lanes_per_step, n_coarse)) {
         a.prefix = scan->prefix;
         a.block_total = scan->block_total;
         scan->blocks = blocks;
@@ -1708,6 +1722,17 @@ size_t ss_evaluate_workspace(int64_t n, int dim)
     return n <= kEvaluateBlocks * 256 ? std::max(scan, evaluate_layout(n, dim).bytes) : scan;
 }
 
+size_t ss_module_evaluate_workspace(const ss_module* m, int64_t n, double dt, double dt_out, int lanes_per_step)
+{
+    if (!m || n <= 0) return 0;
+    const double nf = std::floor(dt_out / dt + 0.5);
+    if (lanes_per_step == 0 && nf >= 0 && nf <= 2147483647.0)
+        lanes_per_step = default_launch(m->dim, m->steps, n, int(nf), m->cus, m->single_blocks, m->phased_blocks);
+    // (calls that ss_evaluate refuses need none)
+    if (lanes_per_step > 64 || !leaves_products(lanes_per_step, n)) return ss_state_scan_workspace(n, m->dim);
+    return std::max(ss_state_scan_workspace(n, m->dim), evaluate_layout(n, m->dim).bytes);
+}
+
 int ss_evaluate(const ss_module* m, const double* sweep, int n_sweep, double t0, double dt, double dt_out,
                 int64_t n_coarse, double* time_out, double* u_out, const ss_table* tables, int lanes_per_step,
                 const double* psi0, double* state, double* spin, void* workspace, size_t workspace_bytes,
@@ -1717,7 +1742,8 @@ int ss_evaluate(const ss_module* m, const double* sweep, int n_sweep, double t0,
         (void)take_te_events();
         return fail("ss_evaluate: 0 to %d sweep parameters in host memory, got %d", SS_SWEEP_INLINE, n_sweep);
     }
-    // up to kEvaluateBlocks workgroups the integrator does the scan's first pass
+    // where its launch allows (leaves_products) the integrator does the scan's
+    // first pass
     EvaluateScan scan = {};
     double* carry = nullptr;
     if (m && psi0 && state && workspace && n_coarse > 0 && n_coarse <= kEvaluateBlocks * 256) {

@@ -550,7 +550,8 @@ class Simulator:
         if lanes == "auto":
             lanes = self._tuned_lanes(on_device, float(ends[0]), dt, time_step_output, n)
         psi0 = np.ascontiguousarray(np.asarray(state_init, np.complex128).reshape(d))
-        ws_bytes = int(_native.lib().ss_evaluate_workspace(n, d))
+        ws_bytes = int(_native.lib().ss_module_evaluate_workspace(
+            self._module(dev).handle, n, dt, float(time_step_output), int(lanes)))
 
         def run(time, u, state, spin, ws, reader=None):
             """Enqueue time evolution and state scan (device addresses)."""
