@@ -199,8 +199,9 @@ class BatchPlan:
         self.state = torch.empty((total, d), dtype=torch.complex128, device=dev)
         self.lanes = int(lanes_per_step or sim.lanes_per_step or 0)
         if self.lanes <= 0:
-            self.lanes = default_batch_lanes(total, int(nf.max(initial=1)),
-                                             sim.precision in ("fp32", "fp32_bulk"))
+            self.lanes = default_batch_lanes(
+                total, int(nf.max(initial=1)), sim.precision in ("fp32", "fp32_bulk"),
+                torch.cuda.get_device_properties(dev).multi_processor_count)
         self.items_per_grab = int(items_per_grab or default_batch_items(total, self.lanes))
         self.grid_blocks = int(grid_blocks)
         self.graph = None
@@ -290,12 +291,15 @@ class BatchPlan:
         return BatchResults(self)
 
 
-def default_batch_lanes(total_rows, max_fine, float32=False):
-    """Lanes per coarse step for a batch: the launch cost model's (256 CUs of
-    three workgroups each).  The float32 modes' results depend on where rows
-    are cut; they keep enough lanes for 32 waves per CU."""
+def default_batch_lanes(total_rows, max_fine, float32=False, cus=256):
+    """Lanes per coarse step for a batch: the launch cost model's for `cus` CUs of
+    three workgroups each.  Three also where a kernel's registers allow two: with
+    those in the model 40 shapes of 25,600 to 300,000 rows of 10 to 100 steps
+    (spin one with a quadratic shift, four callbacks) take 0.83 to 1.20 times as
+    long, 1.01 on average.  The float32 modes' results depend on where rows are
+    cut; they keep enough lanes for 32 waves on each of 256 CUs."""
     if not float32:
-        return int(_native.lib().ss_default_lanes(max(1, int(total_rows)), int(max_fine), 256, 3))
+        return int(_native.lib().ss_default_lanes(max(1, int(total_rows)), int(max_fine), int(cus), 3))
     target = 256 * 4 * 8 * 64
     g = 1
     while g < 64 and 2 * g <= max_fine and total_rows * g < target:
