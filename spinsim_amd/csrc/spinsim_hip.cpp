@@ -159,6 +159,10 @@ constexpr int kSingleScanBlock = 256;
 // workgroups: 17.9 -> 14.8 us; spin one 33.3 -> 29.0).  At the limit each
 // reads 64 (spin one: 144) KiB of totals and the gain is still 18 (11) %.
 constexpr int kFusedScanBlocks = 1024;
+// Spin-half workgroups beyond which the products move by shuffles (wave_scan):
+// at 6e5 rows, 1172 of them, the scan took 37.8 us so and 36.5 without, at 8e5
+// (1563) 47.3 and 47.9, at 2e6 101.9 and 104.9.
+constexpr int kShuffleScanBlocks = 1536;
 // Workgroups up to which ss_evaluate's integrator leaves the products (beyond
 // kFusedScanBlocks one workgroup scans their totals, a few microseconds for each
 // thousand; with several lanes a row its workgroups hold fewer rows, and the
@@ -170,10 +174,26 @@ constexpr long long kEvaluateBlocks = 16384;
 
 // Inclusive scan over the 64 lanes of a wave of x_l (later lanes on the
 // left): q_l = x_l x_{l-1} ... x_0.  Then ex = q_{l-1} (identity on lane 0).
-template <int D>
+// SHUFFLE: moved through the LDS crossbar, which leaves the vector units to the
+// products where many workgroups fill the device (single_scan_lanes of 2e6
+// spin-half rows: 41.3 -> 38.2 us).
+template <int D, bool SHUFFLE = false>
 __device__ __forceinline__ void wave_scan(ss_cd q[D][D], ss_cd ex[D][D], int lane)
 {
-    ss_wave_scan<D>(q, lane, 64);
+    if (SHUFFLE) {
+#pragma unroll 1
+        for (int s = 1; s < 64; s <<= 1) {
+            ss_cd p[D][D];
+#pragma unroll
+            for (int r = 0; r < D; ++r)
+#pragma unroll
+                for (int c = 0; c < D; ++c)
+                    p[r][c] = ss_c(__shfl_up(q[r][c].x, s, 64), __shfl_up(q[r][c].y, s, 64));
+            if (lane >= s) ss_right_multiply<D>(q, p);
+        }
+    } else {
+        ss_wave_scan<D>(q, lane, 64);
+    }
     ss_dpp_mat<D, SS_DPP_WAVE_SHR1>(q, ex);
     if (lane == 0) ss_set_identity<D>(ex);
 }
@@ -182,7 +202,7 @@ __device__ __forceinline__ void wave_scan(ss_cd q[D][D], ss_cd ex[D][D], int lan
 // the product of the x of all earlier lanes of the workgroup; on the lanes of
 // the last wave `total` is the product over the whole workgroup (that wave's
 // own product times the earlier waves', one more matrix product).
-template <int D>
+template <int D, bool SHUFFLE = false>
 __device__ __forceinline__ void block_scan(const ss_cd x[D][D], ss_cd ex[D][D], ss_cd total[D][D])
 {
     __shared__ ss_cd wave_tot[kSingleScanBlock / 64][D][D];
@@ -191,7 +211,7 @@ __device__ __forceinline__ void block_scan(const ss_cd x[D][D], ss_cd ex[D][D], 
     ss_cd q[D][D];
     ss_copy<D>(x, q);
     ss_cd wex[D][D];
-    wave_scan<D>(q, wex, lane);
+    wave_scan<D, SHUFFLE>(q, wex, lane);
     if (lane == 63) ss_copy<D>(q, wave_tot[wave]);
     __syncthreads();
     ss_cd pre[D][D];
@@ -204,7 +224,7 @@ __device__ __forceinline__ void block_scan(const ss_cd x[D][D], ss_cd ex[D][D], 
 // Single simulation, pass 1: lane L covers states [L*C, L*C + C) and the matrices it applies,
 // [L*C, min(L*C + C, n - 1)).  Store each lane's exclusive in-block prefix and
 // each block's total.
-template <int D>
+template <int D, bool SHUFFLE = false>
 __global__ void __launch_bounds__(kSingleScanBlock) single_scan_lanes(const double* u, long long n, double* lane_prefix,
                                                            double* block_total)
 {
@@ -219,7 +239,7 @@ __global__ void __launch_bounds__(kSingleScanBlock) single_scan_lanes(const doub
         ss_left_multiply<D>(m, x);
     }
     ss_cd ex[D][D], total[D][D];
-    block_scan<D>(x, ex, total);
+    block_scan<D, SHUFFLE>(x, ex, total);
     store_mat<D>(lane_prefix, lane_id, ex);
     if (threadIdx.x == kSingleScanBlock - 1) store_mat<D>(block_total, blockIdx.x, total);
 }
@@ -1953,11 +1973,15 @@ int ss_state_scan(const double* psi0, const double* u, double* state, double* sp
     // from the block totals; beyond, one workgroup scans them first
     const bool fused = l.blocks <= kFusedScanBlocks;
     if (dim == 2) {
-        hipLaunchKernelGGL(single_scan_lanes<2>, grid, block, 0, s, u, (long long)n, prefix, total);
         if (fused) {
+            hipLaunchKernelGGL(single_scan_lanes<2>, grid, block, 0, s, u, (long long)n, prefix, total);
             hipLaunchKernelGGL(single_scan_apply_carry<2>, grid, block, 0, s, u, (long long)n, prefix, total, p0,
                                p1, p2, state, spin);
         } else {
+            if (l.blocks > kShuffleScanBlocks)
+                hipLaunchKernelGGL((single_scan_lanes<2, true>), grid, block, 0, s, u, (long long)n, prefix, total);
+            else
+                hipLaunchKernelGGL(single_scan_lanes<2>, grid, block, 0, s, u, (long long)n, prefix, total);
             hipLaunchKernelGGL(single_scan_blocks<2>, dim3(1), block, 0, s, total, l.blocks, p0, p1, p2, carry);
             hipLaunchKernelGGL(single_scan_apply<2>, grid, block, 0, s, u, (long long)n, prefix, carry, state,
                                spin);
