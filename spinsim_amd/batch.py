@@ -190,9 +190,10 @@ class BatchPlan:
         self.offsets_host = offsets
         self.fine_steps = int((n * nf.astype(np.int64)).sum())
         f64 = torch.float64
-        (self.sweep, self.offsets, self.t0, self.dt, self.dt_out, self.n_fine,
-         self.psi0) = _upload(torch, dev, [sweep, offsets, t0, dt, dto, nf, psi])
-        self.counter = self.offsets  # (the launch's counter argument is not used)
+        # (the launch takes a counter, and neither reads nor writes it)
+        (self.sweep, self.offsets, self.t0, self.dt, self.dt_out, self.n_fine, self.psi0,
+         self.counter) = _upload(torch, dev, [sweep, offsets, t0, dt, dto, nf, psi,
+                                              np.zeros(1, np.int64)])
         self.time = torch.empty(total, dtype=f64, device=dev)
         self.u = torch.empty((total, 2) if compact else (total, d, d), dtype=torch.complex128,
                              device=dev)
