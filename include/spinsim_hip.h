@@ -151,7 +151,9 @@ int ss_compile_code(const char *field_src, int dim, int method, int expo, int ro
                     size_t *code_size, char **log);
 void ss_free(void *p);
 
-/* Load a code object from ss_compile_code on the current HIP device. */
+/* Load a code object from ss_compile_code on the current HIP device.  One whose
+ * kernels take other arguments (compiled by another version of this library) is
+ * refused. */
 int ss_module_load(const void *code, size_t code_size, int dim, int method, int expo,
                    int rotating, ss_module **out);
 /* ss_compile_code + ss_module_load. */

@@ -1466,7 +1466,7 @@ static __device__ __forceinline__ void ss_store(ss_cd u[SS_D][SS_D], double rot,
 #ifndef SS_HOST
 // What the host reads from a module: its size, 1, or 2 with float32-bulk step
 // operators.
-extern "C" __device__ __attribute__((used)) char ss_module_traits[SS_PREC == 1 || SS_PREC == 3 ? 2 : 1] = {};
+extern "C" __device__ __attribute__((used)) char SS_MODULE_TRAITS[SS_PREC == 1 || SS_PREC == 3 ? 2 : 1] = {};
 
 // Waves per SIMD the kernels are compiled for at least: the register budget
 // is 512 / waves VGPRs a lane (in 8-register granules).  The time-evolution

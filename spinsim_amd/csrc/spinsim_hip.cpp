@@ -1236,6 +1236,16 @@ ScanLayout scan_layout(int64_t n, int dim, int64_t chunk_rows = 0)
     return l;
 }
 
+// Name of a code object's traits array, by the text of the kernels' arguments: an
+// object for other arguments has no array of this name.
+std::string traits_name()
+{
+    char name[64];
+    snprintf(name, sizeof(name), "ss_module_traits_%016llx",
+             (unsigned long long)fnv1a(ss_src_args, 1469598103934665603ull));
+    return name;
+}
+
 std::string build_source(const char* field_src, int dim, int method, int expo, int rotating,
                          int number_of_squares, int field_has_context, int precision, bool far_inline)
 {
@@ -1261,6 +1271,7 @@ std::string build_source(const char* field_src, int dim, int method, int expo, i
              field_has_context ? 1 : 0,
              precision);
     s += head;
+    s += "#define SS_MODULE_TRAITS " + traits_name() + "\n";
     s += ss_src_args;
     s += ss_src_complex;
     s += ss_src_prelude;
@@ -1459,9 +1470,12 @@ int ss_module_load(const void* code, size_t code_size, int dim, int method, int 
     // (the traits array's size is its content)
     hipDeviceptr_t traits = nullptr;
     size_t traits_size = 0;
-    if (e == hipSuccess && hipModuleGetGlobal(&traits, &traits_size, m->module, "ss_module_traits") != hipSuccess) {
+    if (e == hipSuccess &&
+        hipModuleGetGlobal(&traits, &traits_size, m->module, traits_name().c_str()) != hipSuccess) {
         (void)hipGetLastError();
-        traits_size = SS_STEPS_DIRECT;
+        (void)hipModuleUnload(m->module);
+        delete m;
+        return fail("ss_module_load: a code object of another version of this library (compile the field again)");
     }
     int per_cu = 0, phased_per_cu = 0, cus = 0;
     if (e == hipSuccess) e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m->single, 256, 0);
