@@ -10,6 +10,7 @@ simulation, all stream-ordered and capturable in a HIP graph.
 """
 from __future__ import annotations
 
+import functools
 import math
 
 import numpy as np
@@ -190,19 +191,17 @@ class BatchPlan:
         self.offsets_host = offsets
         self.fine_steps = int((n * nf.astype(np.int64)).sum())
         f64 = torch.float64
-        # (the launch takes a counter, and neither reads nor writes it)
-        (self.sweep, self.offsets, self.t0, self.dt, self.dt_out, self.n_fine, self.psi0,
-         self.counter) = _upload(torch, dev, [sweep, offsets, t0, dt, dto, nf, psi,
-                                              np.zeros(1, np.int64)])
+        (self.sweep, self.offsets, self.t0, self.dt, self.dt_out, self.n_fine,
+         self.psi0) = _upload(torch, dev, [sweep, offsets, t0, dt, dto, nf, psi])
+        self._counter = None
         self.time = torch.empty(total, dtype=f64, device=dev)
         self.u = torch.empty((total, 2) if compact else (total, d, d), dtype=torch.complex128,
                              device=dev)
         self.state = torch.empty((total, d), dtype=torch.complex128, device=dev)
         self.lanes = int(lanes_per_step or sim.lanes_per_step or 0)
         if self.lanes <= 0:
-            self.lanes = default_batch_lanes(
-                total, int(nf.max(initial=1)), sim.precision in ("fp32", "fp32_bulk"),
-                torch.cuda.get_device_properties(dev).multi_processor_count)
+            self.lanes = default_batch_lanes(total, int(nf.max(initial=1)),
+                                             sim.precision in ("fp32", "fp32_bulk"), _cus(dev.index))
         self.items_per_grab = int(items_per_grab or default_batch_items(total, self.lanes))
         self.grid_blocks = int(grid_blocks)
         self.graph = None
@@ -234,6 +233,14 @@ class BatchPlan:
             self.scan_ws = torch.empty(need, dtype=torch.uint8, device=self.device)
         self.scan_chunk_rows = chunk_rows
 
+    @property
+    def counter(self):
+        """One int64, zero at first.  The launch takes a counter's address and neither
+        reads nor writes there (it is given the offsets')."""
+        if self._counter is None:
+            self._counter = self.sim._torch().zeros(1, dtype=self.offsets.dtype, device=self.device)
+        return self._counter
+
     def run_time_evolution(self, stream=None):
         torch = self.sim._torch()
         if stream is None:
@@ -243,7 +250,7 @@ class BatchPlan:
             mod.handle, self.sweep.data_ptr(), self.sweep.shape[1], self.n_sims,
             self.offsets.data_ptr(), self.t0.data_ptr(), self.dt.data_ptr(),
             self.dt_out.data_ptr(), self.n_fine.data_ptr(), self.total, self.time.data_ptr(),
-            self.u.data_ptr(), self.sim._table_ptr(self.device), self.counter.data_ptr(),
+            self.u.data_ptr(), self.sim._table_ptr(self.device), self.offsets.data_ptr(),
             self.lanes, self.items_per_grab, self.grid_blocks, self.u_layout, stream),
             "ss_batch_time_evolution")
 
@@ -290,6 +297,14 @@ class BatchPlan:
 
     def results(self):
         return BatchResults(self)
+
+
+@functools.lru_cache(maxsize=None)
+def _cus(index):
+    """Compute units of a device."""
+    import torch
+
+    return torch.cuda.get_device_properties(index).multi_processor_count
 
 
 def default_batch_lanes(total_rows, max_fine, float32=False, cus=256):
