@@ -141,9 +141,9 @@ uint64_t ss_source_hash(void);
  * per SIMD the time-evolution and adjoint kernels are compiled for; defaults
  * 1 and 2).  dim is 2 (spin half) or 3 (spin one);
  * number_of_squares as in the reference (Lie-Trotter squarings, :1547-1550);
- * precision: SS_PRECISION_*.  The callback's sin and cos resolve to
- * table-driven float64 functions (within 2.3e-16 of the exact values for
- * |x| <= 1e14), with SS_PRECISION_FP32 to float32-evaluated ones (and exp).
+ * precision: SS_PRECISION_*.  The callback's sin, cos and exp resolve to
+ * table-driven float64 functions (sin and cos within 2.3e-16 of the exact values,
+ * exp within 0.51 ulp), with SS_PRECISION_FP32 to float32-evaluated ones.
  * On success *code / *code_size hold a code object and *log the compiler log
  * (both freed with ss_free); on failure *log holds the log when available. */
 int ss_compile_code(const char *field_src, int dim, int method, int expo, int rotating,

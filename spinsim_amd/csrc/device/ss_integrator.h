@@ -1942,8 +1942,8 @@ static __device__ __forceinline__ void ss_adjoint_exp(const double g[SS_FIELD_LE
 // exact for any angle and about 45 instructions, where the two exponentials'
 // series on psi and lambda with the derivative's sums take 460 (the backward
 // kernel of 1024 spin-one pulses of 1e5 steps: 4.7 -> 2.2 ms).  Up to 0.018 rad
-// the series of S2 and S3 stop at theta^4 (below 2e-20 of m), up to 1/2 at
-// theta^12.  Angles that the series of the general case refuses stay refused.
+// the series of S2 and S3 stop at theta^4 (S2's next term, theta^6/40320, leaves
+// out 1.5e-17 of m in dL/dg, S3's 3e-20), up to 1/2 at theta^12.  Angles that the series of the general case refuses stay refused.
 static __device__ __forceinline__ void ss_adjoint_rotate(const double g[SS_FIELD_LEN], double m[3], double d[SS_LIE],
                                                          int* status)
 {
